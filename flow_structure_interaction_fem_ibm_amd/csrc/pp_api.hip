@@ -11,6 +11,7 @@
 #include <rocblas/rocblas.h>
 
 #include "pp_kernels.h"
+#include "pp_momentum.h"
 #include "pp_setup.h"
 
 using namespace pp;
@@ -1625,6 +1626,7 @@ int compute_null_vector(pp_ctx *c) {
 
 void free_fresh_rows(pp_ctx *c) {
   hipFree(c->fr.ids); hipFree(c->fr.face); hipFree(c->fr.coff); hipFree(c->fr.cc);
+  hipFree(c->fr.ids_s); hipFree(c->fr.coff_s);
   c->fr = FreshRows{};
 }
 
@@ -1763,6 +1765,7 @@ int32_t pp_destroy(pp_ctx *c) {
   hipFree(c->d_p); hipFree(c->d_b); hipFree(c->d_w); hipFree(c->d_bwork); hipFree(c->d_tmp);
   hipFree(c->d_fresh); hipFree(c->d_iblank_ref); hipFree(c->d_count); hipFree(c->d_mu); hipFree(c->d_sv);
   hipFree(c->d_ad_coef);
+  hipFree(c->adw.buf);
   hipFree(c->d_nshape32); hipFree(c->d_nshape64);
   free_fresh_rows(c);
   hipFree(c->d_part); hipFree(c->d_part2); hipFree(c->d_res);
@@ -1964,6 +1967,35 @@ int32_t pp_ghost_rows(pp_ctx *c, double *p, const double *bc) {
   return PP_OK;
 }
 
+}  // extern "C"
+
+namespace {
+// the split-row geometry of the momentum solve (csrc/pp_momentum.h): both
+// halves of a row start on a 128-byte line and hold the halo cells
+AdSplit ad_split(const pp_ctx *c) {
+  AdSplit A{};
+  A.cx = c->nxc; A.cy = c->nyc; A.cz = c->nzc;
+  A.hp = ((c->nxc / 2 + 2 + 15) / 16) * 16;
+  A.sx = SPLIT_E0 + 2 * A.hp;
+  A.sxy = (long)A.sx * (c->nyc + 2);
+  A.total = A.sxy * (c->nzc + 2 + kAdMaxLS);
+  double *b = c->adw.buf;
+  for (int q = 0; q < 3; q++) { A.var[q] = b + q * A.total; A.rw[q] = b + (3 + q) * A.total; }
+  A.row = b + 6 * A.total;
+  return A;
+}
+
+// offsets of the reference layout into the momentum solve's split rows
+int ad_split_offsets(pp_ctx *c, int n, const long *ref, long *out) {
+  const AdSplit A = ad_split(c);
+  k_ad_offsets<<<(n + 255) / 256, 256, 0, c->stream>>>(n, c->ref, A.sx, A.sxy, A.hp, ref, out);
+  HIPCHK(hipGetLastError());
+  return PP_OK;
+}
+}  // namespace
+
+extern "C" {
+
 int32_t pp_set_vel_ghosts(pp_ctx *c, const double *coeffD, double bi_weight, double ip_weight) {
   if (!c) { set_error("pp_set_vel_ghosts: null context"); return PP_BAD_ARG; }
   if (!c->have_geom) { set_error("pp_set_vel_ghosts: no geometry (call pp_set_geometry first)"); return PP_NO_GEOMETRY; }
@@ -1975,7 +2007,8 @@ int32_t pp_set_vel_ghosts(pp_ctx *c, const double *coeffD, double bi_weight, dou
   }
   HIPCHK(hipSetDevice(c->device));
   hipFree(g.v_cD); hipFree(g.v_buf[0]); hipFree(g.v_buf[1]); hipFree(g.v_kind); hipFree(g.v_off);
-  g.v_cD = g.v_buf[0] = g.v_buf[1] = nullptr; g.v_kind = nullptr; g.v_off = nullptr;
+  hipFree(g.v_off_s); hipFree(g.g_ref_s);
+  g.v_cD = g.v_buf[0] = g.v_buf[1] = nullptr; g.v_kind = nullptr; g.v_off = g.v_off_s = g.g_ref_s = nullptr;
   g.have_vel = false;
   const int n = g.n;
   std::vector<int> kind(8L * n);
@@ -2039,6 +2072,11 @@ int32_t pp_set_vel_ghosts(pp_ctx *c, const double *coeffD, double bi_weight, dou
     HIPCHK(hipMemcpy(g.v_cD, cd.data(), sizeof(double) * 8 * n, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(g.v_kind, kind.data(), sizeof(int) * 8 * n, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(g.v_off, off.data(), sizeof(long) * 8 * n, hipMemcpyHostToDevice));
+    HIPCHK(hipMalloc(&g.v_off_s, sizeof(long) * 8 * n));
+    HIPCHK(hipMalloc(&g.g_ref_s, sizeof(long) * n));
+    int rc = ad_split_offsets(c, 8 * n, g.v_off, g.v_off_s);
+    if (!rc) rc = ad_split_offsets(c, n, g.g_ref, g.g_ref_s);
+    if (rc) return rc;
   }
   g.v_sweeps = sweeps;
   g.v_bw = bi_weight;
@@ -2052,19 +2090,23 @@ int32_t pp_set_vel_ghosts(pp_ctx *c, const double *coeffD, double bi_weight, dou
 namespace {
 // GCM_vel_set_bc_internal on device fields: gather the ghost cells'
 // (u, v, w), the Jacobi sweeps fixed by pp_set_vel_ghosts, scatter
-void vel_ghosts(pp_ctx *c, double *d_u, double *d_v, double *d_w, const double *d_vbi) {
+// (fields in the momentum solve's split rows when rw is given; the ghosts'
+// new values then go into its masked right-hand sides rw too)
+void vel_ghosts(pp_ctx *c, double *d_u, double *d_v, double *d_w, const double *d_vbi, double *const *rw = nullptr) {
   GhostTables &g = c->gh;
   if (g.n == 0) return;
   hipStream_t s = c->stream;
   dim3 gg((g.n + 255) / 256), blk(256);
-  k_vel_ghost_gather<double><<<gg, blk, 0, s>>>(g.n, g.g_ref, d_u, d_v, d_w, g.v_buf[0]);
+  const long *gref = rw ? g.g_ref_s : g.g_ref, *voff = rw ? g.v_off_s : g.v_off;
+  k_vel_ghost_gather<double><<<gg, blk, 0, s>>>(g.n, gref, d_u, d_v, d_w, g.v_buf[0]);
   int cur = 0;
   for (int q = 0; q < g.v_sweeps; q++) {
-    k_vel_ghost_sweep<<<gg, blk, 0, s>>>(g.n, g.v_cD, g.v_kind, g.v_off, g.v_bw, g.v_iw, d_vbi, d_u, d_v, d_w,
+    k_vel_ghost_sweep<<<gg, blk, 0, s>>>(g.n, g.v_cD, g.v_kind, voff, g.v_bw, g.v_iw, d_vbi, d_u, d_v, d_w,
                                          g.v_buf[cur], g.v_buf[1 - cur]);
     cur ^= 1;
   }
-  k_vel_ghost_scatter<<<gg, blk, 0, s>>>(g.n, g.g_ref, g.v_buf[cur], d_u, d_v, d_w);
+  k_vel_ghost_scatter<<<gg, blk, 0, s>>>(g.n, gref, g.v_buf[cur], d_u, d_v, d_w, rw ? rw[0] : nullptr,
+                                         rw ? rw[1] : nullptr, rw ? rw[2] : nullptr);
 }
 }  // namespace
 
@@ -2605,40 +2647,74 @@ int32_t pp_adjoint(pp_ctx *c, const double *wobj, double *lambda, double *dJ_dg,
 // implicit momentum solve (set_solve_ad, solve_ad, calc_residual_ad)
 // =====================================================================
 namespace {
-// cells per thread of a line segment (x-lines: 2 and 8 measured slower,
-// 31 and 39 ms against 27.5 ms for the 256x192x192 momentum solve)
-constexpr int kAdLS = 4, kAdLSx = 4;
-
 FracMetrics ref_metrics(const pp_ctx *c) {
   FracMetrics M;
   for (int d = 0; d < 3; d++) { M.fx[d] = c->d_rfx[d]; M.dinv[d] = c->d_rdxinv[d]; M.dcinv[d] = c->d_rdxcinv[d]; }
   return M;
 }
 
-struct AdLineLaunch {
-  dim3 grid, block;
-  size_t lds;
-  int nlines;
-};
-// TX lines x P segments per block, TX a power of two up to 32 with at most
-// 512 threads (one segment per thread: P = ceil(n / LS) <= 256)
-AdLineLaunch ad_line_launch(const pp_ctx *c, int dir) {
-  const int n = dir == 0 ? c->nxc : (dir == 1 ? c->nyc : c->nzc);
-  const int ls = dir == 0 ? kAdLSx : kAdLS;
-  const int P = (n + ls - 1) / ls;
-  int tx = 1;
-  while (tx < 32 && 2 * tx * P <= 512) tx *= 2;
-  AdLineLaunch L;
-  L.block = dim3(tx, P);
-  L.lds = sizeof(double) * 12 * (size_t)P * tx;  // seg_reduced_solve_n with 3 right-hand sides
-  if (dir == 0) {
-    L.nlines = ((c->nyc + 1) / 2) * c->nzc;
-    L.grid = dim3((L.nlines + tx - 1) / tx);
-  } else {
-    L.nlines = 0;
-    L.grid = dim3((c->nxc + 2 * tx - 1) / (2 * tx), dir == 1 ? c->nzc : c->nyc);
+// The working copy, allocated at the first call: every value an identity row
+// (coefficients 0, diagonal 1, right-hand side 0) until a solve writes its
+// interior cells.
+int ad_work(pp_ctx *c, AdSplit *out) {
+  AdSplit A = ad_split(c);
+  if (!c->adw.buf) {
+    HIPCHK(hipMalloc(&c->adw.buf, sizeof(double) * 13 * (size_t)A.total));
+    A = ad_split(c);
+    const unsigned nb = 4096;
+    k_fill<double><<<nb, 256, 0, c->stream>>>(c->adw.buf, 12 * A.total, 0.0);
+    k_fill<double><<<nb, 256, 0, c->stream>>>(A.row + 6 * A.total, A.total, 1.0);
+    HIPCHK(hipGetLastError());
   }
-  return L;
+  *out = A;
+  return PP_OK;
+}
+
+// Segment length LS (cells per thread) and tile width TX (lines per block of
+// at most 512 threads) of the y/z passes.  16 lines are one 128-byte line of
+// a half row; 16-cell segments then keep the reduced systems small enough
+// (P = n / 16) that several blocks share a CU (256x192x192: 150 us, 4-cell
+// segments 175; 512x512x384, y: 1538 us, 8-cell segments in 8-line tiles
+// 1604).  Fewer blocks are latency-bound and want short segments: 4 cells
+// below 1024 blocks (130x98x82: 19.1-20.5 us against 19.9-20.5; 96 cells
+// cubed fill half the CUs with 16), 2 cells in 4-line tiles below 256
+// (48x40x32: 4.5-5.0 us against 6.3 with 4 cells in 16-line tiles).
+void ad_yz_shape(int n, int half, int planes, int &LS, int &TX) {
+  const long blocks = (long)((half + 15) / 16) * planes;
+  if (blocks <= 256 && n <= 256) {
+    LS = 2; TX = 4;
+    return;
+  }
+  LS = blocks <= 1024 && n <= 128 ? 4 : kAdMaxLS;
+  TX = 16;
+  while (TX > 1 && TX * ((n + LS - 1) / LS) > 512) TX >>= 1;
+}
+
+template <int DIR>
+void ad_launch_yz(pp_ctx *c, const AdSplit &A, int color) {
+  const int n = DIR == 1 ? A.cy : A.cz, planes = DIR == 1 ? A.cz : A.cy, half = (A.cx + 1) / 2;
+  int LS, TX;
+  ad_yz_shape(n, half, planes, LS, TX);
+  const int P = (n + LS - 1) / LS;
+  const dim3 grid((half + TX - 1) / TX, planes), block(TX, P);
+  const size_t lds = sizeof(double2) * 6 * (size_t)(TX * P + 1);
+  hipStream_t s = c->stream;
+  switch (LS) {
+    case 2: k_ad_yzline<DIR, 2><<<grid, block, lds, s>>>(A, color); break;
+    case 4: k_ad_yzline<DIR, 4><<<grid, block, lds, s>>>(A, color); break;
+    default: k_ad_yzline<DIR, kAdMaxLS><<<grid, block, lds, s>>>(A, color); break;
+  }
+}
+
+// x-lines: blocks of about 256 threads (the same from 64 to 256; 512 cost
+// 16%), 64 where that leaves few blocks (48x40x32: 4.0 against 5.7 us)
+void ad_launch_x(pp_ctx *c, const AdSplit &A, int color) {
+  const int P = (A.cx + 3) / 4;
+  const long lines = (long)((A.cy + 1) / 2) * A.cz;
+  const int nt = lines * P <= 256L * 256 ? 64 : 256;
+  const int TX = std::max(1, nt / P);
+  k_ad_xline<<<(unsigned)((lines + TX - 1) / TX), TX * P, sizeof(double2) * 6 * (size_t)(TX * P + 1), c->stream>>>(
+      A, color, P, TX);
 }
 
 // Fresh cells (fluid now, blank at the previous geometry) take the
@@ -2656,7 +2732,7 @@ FreshRes fresh_res(const pp_ctx *c) {
   if (c->fr.n > 0) {
     r.mask = c->d_fresh;
     r.ids = c->fr.ids;
-    r.coff = c->fr.coff;
+    r.coff = c->fr.coff_s;
     r.cc = c->fr.cc;
     r.n = c->fr.n;
   }
@@ -2670,56 +2746,52 @@ int ad_half_dt(int32_t scheme, double dt, double *half_dt, const char *who) {
   return PP_BAD_ARG;
 }
 
-// the rows of k_ad_rows (7 fields) for the current coefficients
-void ad_build_rows(pp_ctx *c, double half_dt, const double *fu, const double *fv, const double *fw, double *row) {
+// the rows of k_ad_rows for the current coefficients
+void ad_build_rows(pp_ctx *c, const AdSplit &A, double half_dt, const double *fu, const double *fv, const double *fw) {
   CellLaunch cl = ref_launch(c);
   k_ad_rows<256><<<cl.grid, cl.block, 0, c->stream>>>(c->ref, largs<double>(c->lv[0]), ref_metrics(c), half_dt,
-                                                      c->d_ad_coef, fu, fv, fw, c->fr.n > 0 ? c->d_fresh : nullptr,
-                                                      row, c->nref);
+                                                      c->d_ad_coef, c->nref, fu, fv, fw,
+                                                      c->fr.n > 0 ? c->d_fresh : nullptr, A);
 }
 
 // itsolv_ad of u, v and w: x, y and z line sweeps, two zebra passes each
-// (the three fields in each pass); with fresh cells F.r are the call's
-// copies of the right-hand sides that k_fresh_rhs refreshes before each pass
-void ad_sweeps(pp_ctx *c, const double *row, AdLineFields F, const FreshCorr *fc) {
-  LevelArgs<double> L0 = largs<double>(c->lv[0]);
-  for (int dir = 0; dir < 3; dir++) {
-    AdLineLaunch L = ad_line_launch(c, dir);
+// (the three fields in each pass); with fresh cells k_fresh_rhs refreshes
+// their entries of the masked right-hand sides before each pass
+void ad_sweeps(pp_ctx *c, const AdSplit &A, const FreshCorr *fc) {
+  for (int dir = 0; dir < 3; dir++)
     for (int color = 0; color < 2; color++) {
       if (fc)
-        k_fresh_rhs<<<(3 * c->fr.n + 255) / 256, 256, 0, c->stream>>>(c->fr.n, 3, c->fr.ids, c->fr.coff, c->fr.cc,
-                                                                      *fc);
-      if (dir == 0)
-        k_ad_line<0, kAdLSx><<<L.grid, L.block, L.lds, c->stream>>>(c->ref, L0, row, c->nref, F, color, L.nlines);
-      else if (dir == 1)
-        k_ad_line<1, kAdLS><<<L.grid, L.block, L.lds, c->stream>>>(c->ref, L0, row, c->nref, F, color, L.nlines);
-      else
-        k_ad_line<2, kAdLS><<<L.grid, L.block, L.lds, c->stream>>>(c->ref, L0, row, c->nref, F, color, L.nlines);
+        k_fresh_rhs<<<(3 * c->fr.n + 255) / 256, 256, 0, c->stream>>>(c->fr.n, 3, c->fr.ids, c->fr.ids_s,
+                                                                      c->fr.coff_s, c->fr.cc, *fc);
+      if (dir == 0) ad_launch_x(c, A, color);
+      else if (dir == 1) ad_launch_yz<1>(c, A, color);
+      else ad_launch_yz<2>(c, A, color);
     }
-  }
 }
 
-// calc_residual_ad of nv fields: h_res[3q + 1] = max |res|, h_res[3q + 2]
+// u, v, w (or nv = 1 field) and their right-hand sides into the working copy
+template <int NV>
+void ad_copy_in(pp_ctx *c, const AdSplit &A, const AdIn &F) {
+  const int pairs = (c->nxc + 1) / 2 + 1;  // cells -1 .. nxc in pairs (2h - 1, 2h)
+  const int bx = pairs <= 64 ? 64 : (pairs <= 128 ? 128 : 256), by = 256 / bx;
+  const dim3 block(bx, by), grid((pairs + bx - 1) / bx, (c->nyc + 2 + by - 1) / by, c->nzc + 2);
+  k_ad_in<NV><<<grid, block, 0, c->stream>>>(c->ref, largs<double>(c->lv[0]), F, A);
+}
+
+// calc_residual_ad of NV fields: h_res[3q + 1] = max |res|, h_res[3q + 2]
 // = its reference-layout offset (first in k, j, i order), rout the field
 // of the first when not NULL
-int ad_residual(pp_ctx *c, const double *row, int nv, AdFields F, double *rout) {
-  CellLaunch cl = ref_launch(c);
-  const long nblk = c->nblk_red;
-  LevelArgs<double> L0 = largs<double>(c->lv[0]);
+template <int NV>
+int ad_residual(pp_ctx *c, const AdSplit &A, double *rout) {
   hipStream_t s = c->stream;
-  const FreshRes FR = fresh_res(c);
-  if (nv == 3)
-    k_ad_residual<256, 3><<<cl.grid, cl.block, 0, s>>>(c->ref, L0, row, c->nref, F, FR, c->d_part, nblk, rout);
-  else
-    k_ad_residual<256, 1><<<cl.grid, cl.block, 0, s>>>(c->ref, L0, row, c->nref, F, FR, c->d_part, nblk, rout);
-  const int chunk = (int)((nblk + kRedStage - 1) / kRedStage);
-  for (int q = 0; q < nv; q++) {
-    k_reduce_summax_stage<<<kRedStage, 256, 0, s>>>(c->d_part + 3 * nblk * q, (int)nblk, chunk,
-                                                   c->d_part2 + 3 * kRedStage * q);
-    k_reduce_summax<<<1, 256, 0, s>>>(c->d_part2 + 3 * kRedStage * q, kRedStage, c->d_res + 3 * q);
-  }
+  const int pairs = (c->nxc + 1) / 2, kb = c->nzc >= 128 ? 4 : 1;
+  CellLaunch cl = cell_launch(pairs, c->nyc, (c->nzc + kb - 1) / kb);
+  const long nblk = (long)cl.grid.x * cl.grid.y * cl.grid.z;
+  k_ad_residual<256, NV><<<cl.grid, cl.block, 0, s>>>(c->ref, largs<double>(c->lv[0]), A, fresh_res(c), c->d_part, nblk,
+                                                      rout, kb);
+  k_ad_residual_max<<<NV, 1024, 0, s>>>(c->d_part, (int)nblk, c->d_res);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(c->h_res, c->d_res, 3 * nv * sizeof(double), hipMemcpyDeviceToHost, s));
+  HIPCHK(hipMemcpyAsync(c->h_res, c->d_res, 3 * NV * sizeof(double), hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
   return PP_OK;
 }
@@ -2819,6 +2891,11 @@ int32_t pp_set_fresh_cells(pp_ctx *c, int32_t n, const int32_t *ifr, const int32
   HIPCHK(hipMemcpy(F.face, h_face.data(), sizeof(double) * 6 * n, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(F.coff, h_coff.data(), sizeof(long) * 4 * n, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(F.cc, h_cc.data(), sizeof(double) * 4 * n, hipMemcpyHostToDevice));
+  HIPCHK(hipMalloc(&F.ids_s, sizeof(long) * n));
+  HIPCHK(hipMalloc(&F.coff_s, sizeof(long) * 4 * n));
+  int rc = ad_split_offsets(c, n, F.ids, F.ids_s);
+  if (!rc) rc = ad_split_offsets(c, 4 * n, F.coff, F.coff_s);
+  if (rc) return rc;
   F.n = n;
   return PP_OK;
 }
@@ -2871,13 +2948,17 @@ struct FaceVelArgs {
   const double *p, *bcxu, *bcyv, *bczw;
 };
 
+// (SPL: u, v, w in the momentum solve's split rows)
+template <bool SPL = false>
 void face_vel_launch(pp_ctx *c, const FaceVelArgs &a, const double *u, const double *v, const double *w, double *fu,
                      double *fv, double *fw) {
   FracMetrics M;
   for (int d = 0; d < 3; d++) { M.fx[d] = c->d_rfx[d]; M.dinv[d] = c->d_rdxinv[d]; M.dcinv[d] = c->d_rdxcinv[d]; }
   CellLaunch cl = ref_launch(c);
-  k_face_vel<256><<<cl.grid, cl.block, 0, c->stream>>>(c->ref, largs<double>(c->lv[0]), M, a.van_kan, a.dt, a.p, u,
-                                                       v, w, a.bcxu, a.bcyv, a.bczw, fu, fv, fw);
+  const AdSplit A = ad_split(c);
+  k_face_vel<256, SPL><<<cl.grid, cl.block, 0, c->stream>>>(c->ref, largs<double>(c->lv[0]), M, a.van_kan, a.dt, a.p,
+                                                            u, v, w, a.bcxu, a.bcyv, a.bczw, fu, fv, fw, A.sx, A.sxy,
+                                                            A.hp);
 }
 
 // The GCM loop of solve_ad (CORE_SOLVE_AD.F90:218-247) on device fields;
@@ -2911,8 +2992,9 @@ int32_t solve_ad_run(pp_ctx *c, int32_t advec_scheme, double *d_u, double *d_v, 
   if (rc) return rc;
   HIPCHK(hipSetDevice(c->device));
   hipStream_t s = c->stream;
-  DevTemp rows;
-  HIPCHK(rows.alloc(sizeof(double) * 7 * (size_t)c->nref));
+  AdSplit A;
+  rc = ad_work(c, &A);
+  if (rc) return rc;
   // the call's timing events, destroyed on every return path
   struct Events {
     hipEvent_t a = nullptr, b = nullptr;
@@ -2922,39 +3004,35 @@ int32_t solve_ad_run(pp_ctx *c, int32_t advec_scheme, double *d_u, double *d_v, 
   HIPCHK(hipEventCreate(&ev.b));
   hipEvent_t e0 = ev.a, e1 = ev.b;
   HIPCHK(hipEventRecord(e0, s));
-  ad_build_rows(c, half_dt, d_fu, d_fv, d_fw, rows.d());
+  ad_build_rows(c, A, half_dt, d_fu, d_fv, d_fw);
   double *vars[3] = {d_u, d_v, d_w};
   const double *rhs[3] = {d_nlu, d_nlv, d_nlw};
-  AdFields F;
-  for (int q = 0; q < 3; q++) { F.var[q] = vars[q]; F.r[q] = rhs[q]; }
-  // fresh cells: the line passes read copies of nlu, nlv, nlw whose fresh
-  // entries carry the off-stencil terms (k_fresh_rhs)
-  DevTemp rw;
+  AdIn in{};
+  for (int q = 0; q < 3; q++) { in.var[q] = vars[q]; in.r[q] = rhs[q]; }
+  ad_copy_in<3>(c, A, in);
+  // fresh cells: their entries of the working right-hand sides carry the
+  // off-stencil terms during the passes (k_fresh_rhs) and nlu, nlv, nlw
+  // alone for the residual
   FreshCorr fc{};
   const bool fresh = c->fr.n > 0;
-  if (fresh) {
-    const size_t nb = sizeof(double) * (size_t)c->nref;
-    HIPCHK(rw.alloc(3 * nb));
-    for (int q = 0; q < 3; q++) {
-      fc.var[q] = vars[q];
-      fc.r[q] = rhs[q];
-      fc.rw[q] = rw.d() + q * c->nref;
-      HIPCHK(hipMemcpyAsync(fc.rw[q], rhs[q], nb, hipMemcpyDeviceToDevice, s));
-    }
+  for (int q = 0; q < 3; q++) {
+    fc.var[q] = A.var[q];
+    fc.r[q] = rhs[q];
+    fc.rw[q] = A.rw[q];
   }
   int it = 0;
   double maxres = 1.0e10, ruvw[3] = {0.0, 0.0, 0.0};
   int32_t loc[3] = {0, 0, 0};
   while (it < itermax && maxres > restol) {
-    AdLineFields LF;
-    for (int q = 0; q < 3; q++) { LF.var[q] = vars[q]; LF.r[q] = fresh ? fc.rw[q] : rhs[q]; }
-    ad_sweeps(c, rows.d(), LF, fresh ? &fc : nullptr);
-    vel_ghosts(c, d_u, d_v, d_w, d_vbi);
+    ad_sweeps(c, A, fresh ? &fc : nullptr);
+    vel_ghosts(c, A.var[0], A.var[1], A.var[2], d_vbi, A.rw);
     if (cn2) {  // face_vel, then the rows of the new face velocities
-      face_vel_launch(c, *cn2, d_u, d_v, d_w, d_fu, d_fv, d_fw);
-      ad_build_rows(c, half_dt, d_fu, d_fv, d_fw, rows.d());
+      face_vel_launch<true>(c, *cn2, A.var[0], A.var[1], A.var[2], d_fu, d_fv, d_fw);
+      ad_build_rows(c, A, half_dt, d_fu, d_fv, d_fw);
     }
-    rc = ad_residual(c, rows.d(), 3, F, nullptr);
+    if (fresh)
+      k_fresh_rhs<<<(3 * c->fr.n + 255) / 256, 256, 0, s>>>(c->fr.n, 3, c->fr.ids, c->fr.ids_s, nullptr, nullptr, fc);
+    rc = ad_residual<3>(c, A, nullptr);
     if (rc) break;
     int qm = 0;
     for (int q = 0; q < 3; q++) {
@@ -2964,6 +3042,11 @@ int32_t solve_ad_run(pp_ctx *c, int32_t advec_scheme, double *d_u, double *d_v, 
     maxres = ruvw[qm];
     ad_loc(c, c->h_res[3 * qm + 1], c->h_res[3 * qm + 2], loc);
     it++;
+  }
+  if (it > 0) {
+    const CellLaunch cl = ref_launch(c);
+    k_ad_out<<<cl.grid, cl.block, 0, s>>>(c->ref, A, AdOut{{d_u, d_v, d_w}});
+    HIPCHK(hipGetLastError());
   }
   HIPCHK(hipEventRecord(e1, s));
   HIPCHK(hipEventSynchronize(e1));
@@ -3125,19 +3208,22 @@ int32_t pp_calc_residual_ad(pp_ctx *c, int32_t advec_scheme, const double *var, 
   if (rc) return rc;
   HIPCHK(hipSetDevice(c->device));
   const size_t nb = sizeof(double) * c->nref;
-  DevTemp d, rows;
+  DevTemp d;
   HIPCHK(d.alloc(6 * nb));
-  HIPCHK(rows.alloc(7 * nb));
   double *dv[6];
   for (int q = 0; q < 6; q++) dv[q] = d.d() + q * c->nref;
   const double *hin[5] = {var, r, fu, fv, fw};
   for (int q = 0; q < 5; q++) HIPCHK(hipMemcpy(dv[q], hin[q], nb, hipMemcpyHostToDevice));
   HIPCHK(hipMemsetAsync(dv[5], 0, nb, c->stream));
-  ad_build_rows(c, half_dt, dv[2], dv[3], dv[4], rows.d());
-  AdFields F{};
-  F.var[0] = dv[0];
-  F.r[0] = dv[1];
-  rc = ad_residual(c, rows.d(), 1, F, dv[5]);
+  AdSplit A;
+  rc = ad_work(c, &A);
+  if (rc) return rc;
+  ad_build_rows(c, A, half_dt, dv[2], dv[3], dv[4]);
+  AdIn in{};
+  in.var[0] = dv[0];
+  in.r[0] = dv[1];
+  ad_copy_in<1>(c, A, in);
+  rc = ad_residual<1>(c, A, dv[5]);
   if (rc) return rc;
   *resm = c->h_res[1];
   ad_loc(c, c->h_res[1], c->h_res[2], loc);

@@ -149,6 +149,7 @@ struct GhostTables {
   double *v_cD = nullptr, *v_buf[2] = {nullptr, nullptr};
   int *v_kind = nullptr;
   long *v_off = nullptr;
+  long *v_off_s = nullptr, *g_ref_s = nullptr;  // v_off and g_ref in the momentum solve's split rows
   int v_sweeps = 0;                             // Jacobi sweeps that reach round-off
   double v_bw = 0.0, v_iw = 0.0;
   bool have_vel = false;
@@ -161,6 +162,16 @@ struct FreshRows {
   double *face = nullptr;   // 6 per cell: the fresh row's amx_ad..apz_ad
   long *coff = nullptr;     // 4 per cell: offsets of the off-stencil nodes, stencil order
   double *cc = nullptr;     // 4 per cell: their coeffGCMFreshD
+  long *ids_s = nullptr, *coff_s = nullptr;  // ids and coff in the momentum solve's split rows
+};
+
+// The momentum solve's working copy (csrc/pp_momentum.h): u, v, w, their
+// masked right-hand sides and the seven row coefficients in colour-split
+// rows, allocated at the first momentum call and kept with the context.
+struct AdWork {
+  int hp = 0, sx = 0;
+  long sxy = 0, total = 0;     // values per array, spare identity planes included
+  double *buf = nullptr;       // 13 arrays of total values: var 3, rw 3, row 7
 };
 
 // the colour-split copy of level 0 used by the FP32 V-cycles, forward and
@@ -227,6 +238,7 @@ struct pp_ctx {
   double ad_dt = 0.0;
   bool have_ad = false;
   pp::FreshRows fr;                    // fresh-cell rows of the current geometry
+  pp::AdWork adw;                      // working copy of the momentum solve
   int null_iters = 0;
   double null_res = 0.0;           // level-0 smoother uses the transposed ghost rows
   std::vector<double *> d_kry;         // flexible GMRES (FP64 path): m+1 basis + m preconditioned vectors

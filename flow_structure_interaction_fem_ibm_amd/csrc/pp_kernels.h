@@ -481,14 +481,15 @@ __global__ void __launch_bounds__(NT) k_correct_vel(RefArgs R, LevelArgs<double>
 // the west cell's terms only where it is an interior cell.  The cell
 // gradient is the cell's own from fx-interpolated face pressures (the cell
 // value on an outer face).  One thread owns every face it writes.
-template <int NT>
+// SPL: u, v, w in colour-split rows (sidx with pitch vsx, plane vsxy, hp).
+template <int NT, bool SPL>
 __global__ void __launch_bounds__(NT) k_face_vel(RefArgs R, LevelArgs<double> L0, FracMetrics M, int van_kan,
                                                  double dt, const double *__restrict__ p,
                                                  const double *__restrict__ u, const double *__restrict__ v,
                                                  const double *__restrict__ w, const double *__restrict__ bcu,
                                                  const double *__restrict__ bcv, const double *__restrict__ bcw,
                                                  double *__restrict__ fu, double *__restrict__ fv,
-                                                 double *__restrict__ fw) {
+                                                 double *__restrict__ fw, int vsx, long vsxy, int hp) {
 #pragma clang fp contract(off)
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int j = blockIdx.y * blockDim.y + threadIdx.y, k = blockIdx.z;
@@ -503,30 +504,39 @@ __global__ void __launch_bounds__(NT) k_face_vel(RefArgs R, LevelArgs<double> L0
   const uint8_t FM[3] = {FL_IM, FL_JM, FL_KM}, FP[3] = {FL_IP, FL_JP, FL_KP};
   const double *vel[3] = {u, v, w}, *bc[3] = {bcu, bcv, bcw};
   double *face[3] = {fu, fv, fw};
-  // uTilde of the d-component at interior cell q (flags fq, index c along d)
-  auto utilde = [&](int d, long q, uint8_t fq, int c) -> double {
-    if (!van_kan) return vel[d][q];
+  // uTilde of the d-component, value uq, at interior cell q (flags fq, index
+  // c along d)
+  auto utilde = [&](int d, double uq, long q, uint8_t fq, int c) -> double {
+    if (!van_kan) return uq;
     const int mq = (fq & FM[d]) ? 1 : 0, pq = (fq & FP[d]) ? 1 : 0;
     const double fe = M.fx[d][c + 1], fwt = M.fx[d][c], pc = p[q];
     const double pe = (fe * p[q + st[d]] + (1.0 - fe) * pc) * (double)(1 - pq) + pc * (double)pq;
     const double pw = (fwt * pc + (1.0 - fwt) * p[q - st[d]]) * (double)(1 - mq) + pc * (double)mq;
     const double pg = (pe - pw) * M.dinv[d][c];
-    return vel[d][q] + dt * pg * (double)(1 - ((fq & FL_BLANK) ? 1 : 0));
+    return uq + dt * pg * (double)(1 - ((fq & FL_BLANK) ? 1 : 0));
   };
   const bool solid = (f & FL_BLANK) && !(f & FL_GHOST);
   const double gc = (f & FL_GHOST) ? 1.0 : 0.0;
+  // offsets of the velocities of the cell and of its neighbour dn along d
+  auto vat = [&](int d, int dn) -> long {
+    if constexpr (SPL)
+      return sidx(vsx, vsxy, hp, i + (d == 0 ? dn : 0), j + (d == 1 ? dn : 0), k + (d == 2 ? dn : 0));
+    else
+      return id + dn * st[d];
+  };
 #pragma unroll
   for (int d = 0; d < 3; d++) {
     const int c = I[d];
     const int mc = (f & FM[d]) ? 1 : 0, pc = (f & FP[d]) ? 1 : 0;
     const double *U = vel[d];
-    const double uTc = utilde(d, id, f, c);
+    const double uc = U[vat(d, 0)], uw = U[vat(d, -1)];
+    const double uTc = utilde(d, uc, id, f, c);
     // west face
     {
       const bool has_w = c > 1;
       uint8_t fo = 0;
       if (has_w) fo = L0.fl[la - lst[d]];
-      const double uTw = has_w ? utilde(d, id - st[d], fo, c - 1) : U[id - st[d]];
+      const double uTw = has_w ? utilde(d, uw, id - st[d], fo, c - 1) : uw;
       const int pw = (fo & FP[d]) ? 1 : 0;
       const double fxc = M.fx[d][c];
       double x = (fxc * uTc + (1.0 - fxc) * uTw) * (double)(1 - mc) + bc[d][id] * (double)mc;
@@ -541,7 +551,7 @@ __global__ void __launch_bounds__(NT) k_face_vel(RefArgs R, LevelArgs<double> L0
       x = masks(x);
       bool zero = solid;
       if (van_kan) {
-        const double ip = fxc * U[id] + (1.0 - fxc) * U[id - st[d]];
+        const double ip = fxc * uc + (1.0 - fxc) * uw;
         if (has_w) {
           const double gwf = (fo & FL_GHOST) ? 1.0 : 0.0;
           x = (1.0 - gwf) * x + gwf * ip;
@@ -554,7 +564,8 @@ __global__ void __launch_bounds__(NT) k_face_vel(RefArgs R, LevelArgs<double> L0
     // east face of the last cell of a row
     if (c == nc[d]) {
       const double fxe = M.fx[d][c + 1];
-      double x = (fxe * U[id + st[d]] + (1.0 - fxe) * uTc) * (double)(1 - pc) + bc[d][id] * (double)pc;
+      const double ue = U[vat(d, 1)];
+      double x = (fxe * ue + (1.0 - fxe) * uTc) * (double)(1 - pc) + bc[d][id] * (double)pc;
       if (van_kan) {
         const double ge = (p[id + st[d]] - p[id]) * M.dcinv[d][c + 1];
         x = x - dt * ge * (double)(1 - pc);
@@ -562,7 +573,7 @@ __global__ void __launch_bounds__(NT) k_face_vel(RefArgs R, LevelArgs<double> L0
       }
       x = x * (double)(1 - pc) + bc[d][id] * (double)pc;
       if (van_kan) {
-        const double ip = fxe * U[id + st[d]] + (1.0 - fxe) * U[id];
+        const double ip = fxe * ue + (1.0 - fxe) * uc;
         x = (1.0 - gc) * x + gc * ip;
       }
       face[d][id + st[d]] = solid ? 0.0 : x;
@@ -614,12 +625,15 @@ __global__ void k_vel_ghost_sweep(int n, const double *__restrict__ cD, const in
   gout[3L * q + 2] = wb * bw - sw * iw;
 }
 
+// (u2, v2, w2, when given, take the same values)
 __global__ void k_vel_ghost_scatter(int n, const long *__restrict__ gref, const double *__restrict__ g,
-                                    double *__restrict__ u, double *__restrict__ v, double *__restrict__ w) {
+                                    double *__restrict__ u, double *__restrict__ v, double *__restrict__ w,
+                                    double *__restrict__ u2, double *__restrict__ v2, double *__restrict__ w2) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= n) return;
   const long r = gref[q];
   u[r] = g[3 * q]; v[r] = g[3 * q + 1]; w[r] = g[3 * q + 2];
+  if (u2) { u2[r] = g[3 * q]; v2[r] = g[3 * q + 1]; w2[r] = g[3 * q + 2]; }
 }
 
 // update_pressure (CORE_FRAC_STEP_ROUTINES.F90:958-962) over the whole
@@ -2491,52 +2505,6 @@ __global__ void __launch_bounds__(NT) k_set_solve_ad(RefArgs R, LevelArgs<double
   }
 }
 
-// The operator of one cell as itsolv_ad_* and calc_residual_ad build it
-// before masking (CORE_SOLVE_AD.F90:391-421): the viscous coefficients
-// plus the Crank-Nicolson advection terms (half_dt = 0 for
-// ADAMS_BASHFORTH2), and the diagonal sum acx + acy + acz.  Face
-// velocities are fixed during one solve_ad call, so the rows are built
-// once per call: row = amx, apx, amy, apy, amz, apz, sum (nref apart).
-template <int NT>
-__global__ void __launch_bounds__(NT) k_ad_rows(RefArgs R, LevelArgs<double> L0, FracMetrics M, double half_dt,
-                                                const double *__restrict__ coef, const double *__restrict__ fu,
-                                                const double *__restrict__ fv, const double *__restrict__ fw,
-                                                const int8_t *__restrict__ fresh, double *__restrict__ row,
-                                                long nref) {
-#pragma clang fp contract(off)
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int j = blockIdx.y * blockDim.y + threadIdx.y, k = blockIdx.z;
-  if (i >= R.nxc || j >= R.nyc) return;
-  const long id = ridx(R, i, j, k);
-  const uint8_t f = L0.fl[lidx(L0.sx, L0.sxy, i, j, k)];
-  const long st[3] = {1, R.ex, R.exy};
-  const int I[3] = {i + 1, j + 1, k + 1};
-  const uint8_t FM[3] = {FL_IM, FL_JM, FL_KM}, FP[3] = {FL_IP, FL_JP, FL_KP};
-  const double *face[3] = {fu, fv, fw};
-  double ac[3];
-#pragma unroll
-  for (int d = 0; d < 3; d++) {
-    const int um = (f & FM[d]) ? 1 : 0, up = (f & FP[d]) ? 1 : 0;
-    const int q = I[d];
-    double am = coef[(2 * d) * nref + id], ap = coef[(2 * d + 1) * nref + id];
-    double a = -(am + ap);
-    const double fm = M.fx[d][q], fp = M.fx[d][q + 1], di = M.dinv[d][q];
-    const double vm = face[d][id], vp = face[d][id + st[d]];
-    double t1 = 1.0 - fm, t2 = fp;
-    am = am - half_dt * vm * t1 * di;
-    ap = ap + half_dt * vp * t2 * di;
-    t1 = fm * (double)(1 - um);
-    t2 = (1.0 - fp) * (double)(1 - up);
-    a = a + half_dt * (vp * t2 - vm * t1) * di;
-    row[(2 * d) * nref + id] = am;
-    row[(2 * d + 1) * nref + id] = ap;
-    ac[d] = a;
-  }
-  // killForGCMFresh: a fresh cell's diagonal is 1 (CORE_SOLVE_AD.F90:425-427, 866)
-  const double kill = fresh ? 1.0 - 1.0 * (double)fresh[id] : 1.0;
-  row[6 * nref + id] = (ac[0] + ac[1] + ac[2]) * kill;
-}
-
 // Fresh-cell rows of set_solve_ad's GCM branch (CORE_SET_SOLVERS.F90:
 // 175-218): amx_ad..apz_ad of each fresh cell replaced by -coeffGCMFreshD of
 // its face neighbour in the stencil, 0 where the stencil has none (face: 6
@@ -2554,24 +2522,27 @@ __global__ void k_fresh_ad_coef(int n, const long *__restrict__ ids, const doubl
 // for a zebra line pass: rw = r + sum_m cc_m var(coff_m) at each fresh cell
 // (the four stencil nodes that differ from the cell in two or more indices,
 // in stencil order), from the fields as the pass starts, so every line of
-// the pass reads the same values.  rw is the call's copy of r, equal to r
-// off the fresh cells.  One thread per cell and field.
+// the pass reads the same values.  var and rw are the momentum solve's split
+// rows (offsets ids_s, coff), r the caller's fields (offsets ids); coff null:
+// rw = r alone.  One thread per cell and field.
 struct FreshCorr {
   const double *var[3];
   const double *r[3];
   double *rw[3];
 };
-__global__ void k_fresh_rhs(int n, int nv, const long *__restrict__ ids, const long *__restrict__ coff,
-                            const double *__restrict__ cc, FreshCorr F) {
+__global__ void k_fresh_rhs(int n, int nv, const long *__restrict__ ids, const long *__restrict__ ids_s,
+                            const long *__restrict__ coff, const double *__restrict__ cc, FreshCorr F) {
 #pragma clang fp contract(off)
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n * nv) return;
   const int q = t % n, f = t / n;
   const double *var = F.var[f];
   double s = 0.0;
+  if (coff) {
 #pragma unroll
-  for (int m = 0; m < 4; m++) s = s + cc[4 * q + m] * var[coff[4 * q + m]];
-  F.rw[f][ids[q]] = F.r[f][ids[q]] + s;
+    for (int m = 0; m < 4; m++) s = s + cc[4 * q + m] * var[coff[4 * q + m]];
+  }
+  F.rw[f][ids_s[q]] = F.r[f][ids[q]] + s;
 }
 
 // index of reference offset id in the ascending fresh list, -1 if absent
@@ -2632,192 +2603,6 @@ struct SegElimN {
   }
 };
 
-// seg_reduced_solve for SegElimN: the reduced matrix (A, B, C) once, NR
-// right-hand sides R; LDS [buf][seg][field][tx] with 3 + NR fields
-// (2 * (3 + NR) * P * blockDim.x elements).  Every thread of the block must
-// call it.
-template <typename T, int LS, int NR>
-__device__ inline void seg_reduced_solve_n(T *sh, int P, int tx, int seg, SegElimN<T, LS, NR> &se, T (&XL)[NR],
-                                           T (&XS)[NR]) {
-  constexpr int NF = 3 + NR;
-  T cl, dl[NR], fl;
-  se.back(cl, dl, fl);
-  const int TXb = blockDim.x;
-  T *bufA = sh, *bufB = sh + NF * TXb * P;
-  auto E_ = [&](T *buf, int s, int fld) -> T & { return buf[((long)s * NF + fld) * TXb + tx]; };
-#pragma unroll
-  for (int q = 0; q < NR; q++) E_(bufB, seg, q) = se.dp[q][0];
-  E_(bufB, seg, NR) = se.fp[0]; E_(bufB, seg, NR + 1) = se.cp[0];
-  __syncthreads();
-  T D0n[NR], F0n = T(0), G0n = T(0);
-#pragma unroll
-  for (int q = 0; q < NR; q++) D0n[q] = T(0);
-  if (seg + 1 < P) {
-#pragma unroll
-    for (int q = 0; q < NR; q++) D0n[q] = E_(bufB, seg + 1, q);
-    F0n = E_(bufB, seg + 1, NR); G0n = E_(bufB, seg + 1, NR + 1);
-  }
-  T A = -fl, B = T(1) + cl * F0n, C = cl * G0n, R[NR];
-#pragma unroll
-  for (int q = 0; q < NR; q++) R[q] = dl[q] - cl * D0n[q];
-  T *cur = bufA, *nxt = bufB;
-  E_(cur, seg, 0) = A; E_(cur, seg, 1) = B; E_(cur, seg, 2) = C;
-#pragma unroll
-  for (int q = 0; q < NR; q++) E_(cur, seg, 3 + q) = R[q];
-  __syncthreads();
-  for (int d = 1; d < P; d <<= 1) {
-    T Am = T(0), Bm = T(1), Cm = T(0), Ap = T(0), Bp = T(1), Cp = T(0), Rm[NR], Rp[NR];
-#pragma unroll
-    for (int q = 0; q < NR; q++) { Rm[q] = T(0); Rp[q] = T(0); }
-    if (seg - d >= 0) {
-      Am = E_(cur, seg - d, 0); Bm = E_(cur, seg - d, 1); Cm = E_(cur, seg - d, 2);
-#pragma unroll
-      for (int q = 0; q < NR; q++) Rm[q] = E_(cur, seg - d, 3 + q);
-    }
-    if (seg + d < P) {
-      Ap = E_(cur, seg + d, 0); Bp = E_(cur, seg + d, 1); Cp = E_(cur, seg + d, 2);
-#pragma unroll
-      for (int q = 0; q < NR; q++) Rp[q] = E_(cur, seg + d, 3 + q);
-    }
-    T k1 = A * fast_rcp(Bm), k2 = C * fast_rcp(Bp);
-    T nA = -Am * k1, nC = -Cp * k2;
-    T nB = B - Cm * k1 - Ap * k2;
-#pragma unroll
-    for (int q = 0; q < NR; q++) R[q] = R[q] - Rm[q] * k1 - Rp[q] * k2;
-    A = nA; B = nB; C = nC;
-    E_(nxt, seg, 0) = A; E_(nxt, seg, 1) = B; E_(nxt, seg, 2) = C;
-#pragma unroll
-    for (int q = 0; q < NR; q++) E_(nxt, seg, 3 + q) = R[q];
-    __syncthreads();
-    T *t = cur; cur = nxt; nxt = t;
-  }
-  const T rB = fast_rcp(B);
-#pragma unroll
-  for (int q = 0; q < NR; q++) {
-    XS[q] = R[q] * rB;
-    E_(nxt, seg, q) = XS[q];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < NR; q++) XL[q] = seg > 0 ? E_(nxt, seg - 1, q) : T(0);
-}
-
-// One zebra pass of the momentum line sweeps along DIR (0 x, 1 y, 2 z)
-// for u, v and w together: the three share the row coefficients, which are
-// read once, and are independent until the ghost update, so solving them
-// in one pass gives what three passes would.  Lines of colour `color` (the
-// parity of the sum of their two transverse indices), so every off-line
-// neighbour has the other colour and the pass is deterministic.  A block
-// of TX lines x P segments of LS cells; each thread eliminates its segment
-// of the three fields in registers (one elimination of the shared matrix)
-// and the reduced system of a line is solved by cyclic reduction in LDS
-// with three right-hand sides (seg_reduced_solve_n).  For
-// x-lines the segments of one line are adjacent lanes (coalesced along the
-// row); for y- and z-lines adjacent lanes are every other i.
-// Row of a cell (itsolv_ad_x/y/z): off-line terms subtracted from r in the
-// reference's grouping, masked line coefficients, diagonal
-// 1 + sum * (1 - iblank), right-hand side r' (1 - iblank) + var * ghost.
-struct AdLineFields {
-  double *var[3];
-  const double *r[3];
-};
-template <int DIR, int LS>
-__global__ void __launch_bounds__(512) k_ad_line(RefArgs R, LevelArgs<double> L0, const double *__restrict__ row,
-                                                 long nref, AdLineFields F, int color, int nlines) {
-#pragma clang fp contract(off)
-  extern __shared__ unsigned char smem_raw[];
-  double *sh = reinterpret_cast<double *>(smem_raw);
-  const int TX = blockDim.x, P = blockDim.y;
-  int tx, seg, i = 0, j = 0, k = 0;
-  bool ok;
-  if (DIR == 0) {
-    const int flat = threadIdx.x + threadIdx.y * TX;
-    seg = flat % P;
-    tx = flat / P;
-    const int line = blockIdx.x * TX + tx;
-    const int nyh = (R.nyc + 1) >> 1;
-    k = line / nyh;
-    j = 2 * (line - k * nyh) + ((k + color) & 1);
-    ok = line < nlines && k < R.nzc && j < R.nyc;
-  } else {
-    tx = threadIdx.x;
-    seg = threadIdx.y;
-    const int plane = blockIdx.y;
-    i = 2 * (blockIdx.x * TX + tx) + ((plane + color) & 1);
-    if (DIR == 1) k = plane; else j = plane;
-    ok = i < R.nxc && plane < (DIR == 1 ? R.nzc : R.nyc);
-  }
-  const int n = DIR == 0 ? R.nxc : (DIR == 1 ? R.nyc : R.nzc);
-  const long rst = DIR == 0 ? 1 : (DIR == 1 ? R.ex : R.exy);
-  const long lst = DIR == 0 ? 1 : (DIR == 1 ? (long)L0.sx : L0.sxy);
-  const int m0 = seg * LS;
-  long id0 = 0, la0 = 0;
-  if (ok) {
-    const int i0 = DIR == 0 ? m0 : i, j0 = DIR == 1 ? m0 : j, k0 = DIR == 2 ? m0 : k;
-    id0 = ridx(R, i0, j0, k0);
-    la0 = lidx(L0.sx, L0.sxy, i0, j0, k0);
-  }
-  SegElimN<double, LS, 3> se;
-#pragma unroll
-  for (int m = 0; m < LS; m++) {
-    double a = 0.0, b = 1.0, c = 0.0, d[3] = {0.0, 0.0, 0.0};
-    if (ok && m0 + m < n) {
-      const long id = id0 + m * rst;
-      const uint8_t f = L0.fl[la0 + m * lst];
-      const double rib = (f & FL_BLANK) ? 0.0 : 1.0;
-      const double gh = (f & FL_GHOST) ? 1.0 : 0.0;
-      const double amx = row[id], apx = row[nref + id], amy = row[2 * nref + id], apy = row[3 * nref + id];
-      const double amz = row[4 * nref + id], apz = row[5 * nref + id], sum = row[6 * nref + id];
-      const double oim = (f & FL_IM) ? 0.0 : 1.0, oip = (f & FL_IP) ? 0.0 : 1.0;
-      const double ojm = (f & FL_JM) ? 0.0 : 1.0, ojp = (f & FL_JP) ? 0.0 : 1.0;
-      const double okm = (f & FL_KM) ? 0.0 : 1.0, okp = (f & FL_KP) ? 0.0 : 1.0;
-      if (DIR == 0) {
-        a = amx * rib * oim;
-        c = apx * rib * oip;
-      } else if (DIR == 1) {
-        a = amy * rib * ojm;
-        c = apy * rib * ojp;
-      } else {
-        a = amz * rib * okm;
-        c = apz * rib * okp;
-      }
-      b = 1.0 + sum * rib;
-#pragma unroll
-      for (int q = 0; q < 3; q++) {
-        const double *var = F.var[q];
-        double rhs;
-        if (DIR == 0)
-          rhs = F.r[q][id] - (var[id - R.ex] * amy * ojm + var[id + R.ex] * apy * ojp +
-                              var[id - R.exy] * amz * okm + var[id + R.exy] * apz * okp);
-        else if (DIR == 1)
-          rhs = F.r[q][id] - (var[id - 1] * amx * oim + var[id + 1] * apx * oip + var[id - R.exy] * amz * okm +
-                              var[id + R.exy] * apz * okp);
-        else
-          rhs = F.r[q][id] - var[id - R.ex] * amy * ojm - var[id + R.ex] * apy * ojp - var[id - 1] * amx * oim -
-                var[id + 1] * apx * oip;
-        d[q] = rhs * rib + var[id] * gh;
-      }
-    }
-    se.push(m, a, b, c, d);
-  }
-  double XL[3], XS[3];
-  seg_reduced_solve_n<double, LS, 3>(sh, P, tx, seg, se, XL, XS);
-  if (!ok) return;
-#pragma unroll
-  for (int q = 0; q < 3; q++) {
-    se.combine(q, XL[q], XS[q]);
-#pragma unroll
-    for (int m = 0; m < LS; m++)
-      if (m0 + m < n) F.var[q][id0 + m * rst] = se.dp[q][m];
-  }
-}
-
-// calc_residual_ad for NV fields (u, v, w share the rows): per-block
-// partials (0, max |res|, argmax) of each field at part + 3*nblk*q, the
-// argmax the smallest reference-layout offset of the block's maximum.
-struct AdFields {
-  const double *var[3], *r[3];
-};
 // fresh cells of the residual: mask (reference layout, NULL = none), the
 // ascending offsets and the four off-stencil nodes and weights of each
 struct FreshRes {
@@ -2826,55 +2611,4 @@ struct FreshRes {
   const double *cc;
   int n;
 };
-template <int NT, int NV>
-__global__ void __launch_bounds__(NT) k_ad_residual(RefArgs R, LevelArgs<double> L0, const double *__restrict__ row,
-                                                    long nref, AdFields F, FreshRes FR, double *__restrict__ part,
-                                                    long nblk, double *__restrict__ rout) {
-#pragma clang fp contract(off)
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int j = blockIdx.y * blockDim.y + threadIdx.y, k = blockIdx.z;
-  const bool in = i < R.nxc && j < R.nyc;
-  long id = 0;
-  uint8_t f = FL_BLANK;
-  double amx = 0, apx = 0, amy = 0, apy = 0, amz = 0, apz = 0, sum = 0;
-  if (in) {
-    id = ridx(R, i, j, k);
-    f = L0.fl[lidx(L0.sx, L0.sxy, i, j, k)];
-    amx = row[id]; apx = row[nref + id]; amy = row[2 * nref + id]; apy = row[3 * nref + id];
-    amz = row[4 * nref + id]; apz = row[5 * nref + id]; sum = row[6 * nref + id];
-  }
-  const double oim = (f & FL_IM) ? 0.0 : 1.0, oip = (f & FL_IP) ? 0.0 : 1.0;
-  const double ojm = (f & FL_JM) ? 0.0 : 1.0, ojp = (f & FL_JP) ? 0.0 : 1.0;
-  const double okm = (f & FL_KM) ? 0.0 : 1.0, okp = (f & FL_KP) ? 0.0 : 1.0;
-  const double fl = (f & FL_BLANK) ? 0.0 : 1.0;
-  // GCM_correct_res_ad (GCM_FRESHCELL_AD.F90:73-137): the off-stencil terms
-  // of a fresh cell, added one by one in stencil order before the iblank mask
-  const int fq = (in && FR.mask && FR.mask[id]) ? fresh_find(FR.ids, FR.n, id) : -1;
-  const long blk = blockIdx.x + (long)gridDim.x * (blockIdx.y + (long)gridDim.y * blockIdx.z);
-#pragma unroll
-  for (int q = 0; q < NV; q++) {
-    SumMax v{0.0, 0.0, -1};
-    if (in) {
-      const double *x = F.var[q];
-      double s = F.r[q][id] - x[id] * (1.0 + sum * 1.0) - x[id - 1] * amx * oim - x[id + 1] * apx * oip -
-                 x[id - R.ex] * amy * ojm - x[id + R.ex] * apy * ojp - x[id - R.exy] * amz * okm -
-                 x[id + R.exy] * apz * okp;
-      if (fq >= 0)
-        for (int m = 0; m < 4; m++) s = s + FR.cc[4 * fq + m] * x[FR.coff[4 * fq + m]];
-      s = s * fl;
-      if (rout) rout[id] = s;
-      v.mx = fabs(s);
-      v.arg = id;
-    }
-    v = block_summax<NT>(v);
-    if (threadIdx.x == 0 && threadIdx.y == 0) {
-      double *pq = part + 3 * nblk * q;
-      pq[3 * blk] = 0.0;
-      pq[3 * blk + 1] = v.mx;
-      pq[3 * blk + 2] = (double)v.arg;
-    }
-    __syncthreads();
-  }
-}
-
 }  // namespace pp
