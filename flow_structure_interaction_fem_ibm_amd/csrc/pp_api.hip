@@ -267,81 +267,60 @@ void launch_xline(pp_ctx *c, Level &L, int lvl, int color, T omega) {
   kend(c);
 }
 
-// segment length LS and segments P for a line of n cells
-// FP32: up to 16 segments of up to 16 cells (64 x P threads); FP64 keeps
-// at most 12 cells per thread in registers and uses up to 32 segments
-// (32 x P threads) for long lines.
-void yz_shape(int n, int &LS, int &P, int &TX, int elem = 4) {
-  // at most 8 cells per thread (FP64 register budget; FP32 measured no
-  // faster with 12 or 16), at most 16 segments while that suffices
-  static const int opts[] = {1, 2, 4, 8};
-  int maxls = 8;
-  LS = maxls;
-  for (int o : opts) {
-    if ((n + o - 1) / o <= 16) { LS = o; break; }
+// Shape of a y/z pass over lines of n cells (half of them per row, planes
+// rows): LS cells per thread, P segments, TX lines per block (at most 1024
+// threads in FP32, 512 in FP64, whose segments take twice the registers).
+// A wide tile is one 128-byte line of a half row.  Longer segments cost fewer
+// reduction steps and barriers per cell, so LS is the longest that fills the
+// block and still lets the level's blocks be resident at once or nearly so:
+// 12 up to 192 cells (256x192x192 15.6 us; 16: 18.9, 8: 16.7), 16 beyond
+// (384x256x256 42 us; 8: 43, 12: 47; 512-cell lines 245; 8 in 16-line tiles
+// 262).  Levels of few blocks are latency-bound and get 8-line tiles of short
+// segments (128x96x96: 4 cells 6.3 us, 6 cells 6.6, 8 cells 6.9).
+struct YZShape {
+  int LS, P, TX;
+};
+YZShape yz_shape(int n, int half, int planes, int elem) {
+  YZShape s;
+  const int maxt = elem == 4 ? 1024 : 512;
+  if ((long)((half + 7) / 8) * planes <= 2048) {
+    s.TX = 8;
+    s.LS = n <= 16 ? 1 : (n <= 32 ? 2 : (n <= 128 ? 4 : (n <= 256 ? 8 : 16)));
+  } else {
+    s.TX = elem == 4 ? 32 : 16;
+    s.LS = n <= 128 ? 8 : (n <= 192 ? 12 : 16);
   }
-  P = (n + LS - 1) / LS;
-  // TX x P <= 1024 threads: lines of up to 1024 cells
-  TX = P <= 16 ? 64 : (P <= 32 ? 32 : (P <= 64 ? 16 : 8));
-  (void)elem;
+  s.P = (n + s.LS - 1) / s.LS;
+  while (s.TX * s.P > maxt) s.TX >>= 1;
+  return s;
 }
 
 template <typename T, int DIR>
 void launch_yzline(pp_ctx *c, Level &L, int lvl, int color, T omega) {
-  LevelArgs<T> a = largs<T>(L);
-  int n = DIR == 1 ? L.cy : L.cz;
-  int planes = DIR == 1 ? L.cz : L.cy;
-  int LS, P, TX;
-  yz_shape(n, LS, P, TX, (int)sizeof(T));
-  int half = (L.cx + 1) / 2;
-  // small levels are latency-bound: narrow tiles give more blocks (measured
-  // on 128x96x96 ... 32x24x24: 20-25% faster than 64-line tiles)
-  if ((long)((half + 7) / 8) * planes <= 2048) TX = 8;
-  dim3 grid((half + TX - 1) / TX, planes), block(TX, P);
-  size_t sh = sizeof(T) * 8 * TX * P;
-  T *e = lv_e<T>(L);
-  const T *rhs = lv_rhs<T>(L);
+  const bool spl = split_on<T>(c, lvl);
+  const LevelArgs<T> a = spl ? split_args<T>(c, L) : largs<T>(L);
+  const int half = (L.cx + 1) / 2, planes = DIR == 1 ? L.cz : L.cy;
+  const YZShape sh = yz_shape(DIR == 1 ? L.cy : L.cz, half, planes, (int)sizeof(T));
+  const dim3 grid((half + sh.TX - 1) / sh.TX, planes), block(sh.TX, sh.P);
+  const size_t lds = sizeof(RedEq<T>) * 2 * sh.TX * (sh.P + 1);
+  T *e = spl ? split_e<T>(c) : lv_e<T>(L);
+  const T *rhs = spl ? split_rhs<T>(c) : lv_rhs<T>(L);
+  const int hp = c->sp.hp;
   hipStream_t st = c->stream;
   kbegin(c, DIR == 1 ? PP_K_YLINE : PP_K_ZLINE, lvl, 0.5 * (double)L.cx * L.cy * L.cz * bytes_line(sizeof(T)));
-  if constexpr (std::is_same<T, float>::value) {
-    if (split_on<T>(c, lvl)) {
-      // at most 768 threads per block where tiles of 16 lines allow it: with
-      // the split kernel's register budget (six wavefronts per SIMD) two
-      // blocks then share a CU (narrower tiles cost more in coalescing)
-      if (TX > 8) {
-        TX = 64;
-        while (TX > 16 && TX * P > 768) TX >>= 1;
-        grid = dim3((half + TX - 1) / TX, planes);
-        block = dim3(TX, P);
-        sh = sizeof(T) * 8 * TX * P;
-      }
-      LevelArgs<float> as = split_args<float>(c, L);
-      float *es = c->sp.e;
-      const float *rs = c->sp.rhs;
-      const int hp = c->sp.hp;
-      switch (LS) {
-        case 1: k_yzline_split<1, DIR><<<grid, block, sh, st>>>(as, hp, rs, es, color, omega); break;
-        case 2: k_yzline_split<2, DIR><<<grid, block, sh, st>>>(as, hp, rs, es, color, omega); break;
-        case 4: k_yzline_split<4, DIR><<<grid, block, sh, st>>>(as, hp, rs, es, color, omega); break;
-        default: k_yzline_split<8, DIR><<<grid, block, sh, st>>>(as, hp, rs, es, color, omega); break;
-      }
-      kend(c);
-      return;
-    }
-  }
-  // loads issued up front on the narrow-tile (latency-bound) FP32 levels
-  const bool upf = sizeof(T) == 4 && TX == 8;
-  switch (LS) {
-    case 1: k_yzline<T, 1, DIR><<<grid, block, sh, st>>>(a, rhs, e, color, omega); break;
-    case 2: k_yzline<T, 2, DIR><<<grid, block, sh, st>>>(a, rhs, e, color, omega); break;
-    case 4:
-      if (upf) k_yzline<T, 4, DIR, true><<<grid, block, sh, st>>>(a, rhs, e, color, omega);
-      else k_yzline<T, 4, DIR><<<grid, block, sh, st>>>(a, rhs, e, color, omega);
-      break;
-    default:
-      if (upf) k_yzline<T, 8, DIR, true><<<grid, block, sh, st>>>(a, rhs, e, color, omega);
-      else k_yzline<T, 8, DIR><<<grid, block, sh, st>>>(a, rhs, e, color, omega);
-      break;
+  auto go = [&](auto ls) {
+    constexpr int LS = decltype(ls)::value;
+    if (spl) k_yzline<T, LS, DIR, true><<<grid, block, lds, st>>>(a, hp, rhs, e, color, omega);
+    else k_yzline<T, LS, DIR, false><<<grid, block, lds, st>>>(a, hp, rhs, e, color, omega);
+  };
+  using std::integral_constant;
+  switch (sh.LS) {
+    case 1: go(integral_constant<int, 1>{}); break;
+    case 2: go(integral_constant<int, 2>{}); break;
+    case 4: go(integral_constant<int, 4>{}); break;
+    case 8: go(integral_constant<int, 8>{}); break;
+    case 12: go(integral_constant<int, 12>{}); break;
+    default: go(integral_constant<int, 16>{}); break;
   }
   kend(c);
 }
@@ -2480,10 +2459,11 @@ int32_t pp_tdma_batched(pp_ctx *c, const double *a, const double *b, const doubl
       k_tdma_wave<decltype(g)::value, decltype(sz)::value><<<grid, block, 0, s>>>(n, nl, d[0], d[1], d[2], d[3], d[4]);
     });
   } else {
-    int LS, P, TX;
-    yz_shape(n, LS, P, TX, 8);
+    // at most 8 rows per thread and 16 segments while that suffices
+    const int LS = n <= 16 ? 1 : (n <= 32 ? 2 : (n <= 64 ? 4 : 8)), P = (n + LS - 1) / LS;
+    const int TX = P <= 16 ? 64 : (P <= 32 ? 32 : (P <= 64 ? 16 : 8));
     dim3 grid((nl + TX - 1) / TX), block(TX, P);
-    size_t sh = sizeof(double) * 8 * TX * P;
+    size_t sh = sizeof(RedEq<double>) * 2 * TX * (P + 1);
     switch (LS) {
       case 1: k_tdma_seg<1><<<grid, block, sh, s>>>(n, nl, d[0], d[1], d[2], d[3], d[4]); break;
       case 2: k_tdma_seg<2><<<grid, block, sh, s>>>(n, nl, d[0], d[1], d[2], d[3], d[4]); break;

@@ -1561,9 +1561,14 @@ __device__ inline int xcd_block(int b, int nb) {
 // x-line zebra pass (lines along the contiguous index): lines (j,k) with
 // (j+k)%2 == color; a group of G lanes holds one line, S cells per lane.
 // ---------------------------------------------------------------------
-// SPL: the level is in the colour-split row layout (sidx, half-row offset
-// hp; S even): a lane's S cells are S/2 consecutive even cells and the S/2
-// odd cells beside them.
+// SPL: the level is the finest in the colour-split row layout (sidx,
+// half-row offset hp; S even): a lane's S cells are S/2 consecutive even
+// cells and the S/2 odd cells beside them, read whole (the rows' padding and
+// the coefficients' run past the line's end).  Its faces are closed on the
+// outer boundary only, where the coefficients are 0, so its rows test the
+// blank flag alone; rows are chosen by selects, without branches: 256x192x192
+// 16.6 us per colour pass (FP64 32.1) against 20.6 (41.7) with a branch per
+// cell and flag, 467 against 917 VALU instructions per wavefront.
 template <typename T, int G, int S, bool SPL = false>
 __global__ void __launch_bounds__(256) k_xline(LevelArgs<T> L, const T *__restrict__ rhs, T *__restrict__ e,
                                                int color, T omega, int hp) {
@@ -1572,123 +1577,156 @@ __global__ void __launch_bounds__(256) k_xline(LevelArgs<T> L, const T *__restri
   const int line = (blk * 256 + (int)threadIdx.x) / G;
   const int sub = threadIdx.x & (G - 1);
   const int nyh = (L.cy + 1) >> 1;
-  const int k = line / nyh;
-  const int j = 2 * (line - k * nyh) + ((k + color) & 1);
-  const bool valid = k < L.cz && j < L.cy;
+  const int kl = line / nyh;
+  const int jl = 2 * (line - kl * nyh) + ((kl + color) & 1);
+  const bool valid = kl < L.cz && jl < L.cy;
+  const int j = valid ? jl : 0, k = valid ? kl : 0;  // lanes past the level read its first line
   const int i0 = sub * S;
-  const int nv = valid ? max(0, min(S, L.cx - i0)) : 0;
-  const long base = valid ? (SPL ? sidx(L.sx, L.sxy, hp, i0, j, k) : lidx(L.sx, L.sxy, i0, j, k)) : 0;
-  T eo[S], ejm[S], ejp[S], ekm[S], ekp[S], rv[S], cmx[S], cpx[S];
+  const int nv = max(0, min(S, L.cx - i0));
+  const long base = SPL ? sidx(L.sx, L.sxy, hp, i0, j, k) : lidx(L.sx, L.sxy, i0, j, k);
+  T eo[S], rv[S], cmx[S], cpx[S];
   uint8_t fl[S];
   auto ld = [&](const T *p, T(&v)[S]) {
     if constexpr (SPL) {
       T a[S / 2], b[S / 2];
-      load_chunk<T, S / 2>(p, (nv + 1) >> 1, a);
-      load_chunk<T, S / 2>(p + hp, nv >> 1, b);
+      load_chunk<T, S / 2>(p, S / 2, a);
+      load_chunk<T, S / 2>(p + hp, S / 2, b);
 #pragma unroll
       for (int q = 0; q < S / 2; q++) { v[2 * q] = a[q]; v[2 * q + 1] = b[q]; }
     } else {
       load_chunk<T, S>(p, nv, v);
     }
   };
+  const T my = L.cmy[j], py = L.cpy[j], mz = L.cmz[k], pz = L.cpz[k];
   ld(e + base, eo);
-  ld(e + base - L.sx, ejm);
-  ld(e + base + L.sx, ejp);
-  ld(e + base - L.sxy, ekm);
-  ld(e + base + L.sxy, ekp);
   ld(rhs + base, rv);
-  load_chunk<T, S>(L.cmx + i0, nv, cmx);
-  load_chunk<T, S>(L.cpx + i0, nv, cpx);
-  if constexpr (SPL) {
-    uint8_t a[S / 2], b[S / 2];
-    load_flags<S / 2>(L.fl + base, (nv + 1) >> 1, a);
-    load_flags<S / 2>(L.fl + base + hp, nv >> 1, b);
-#pragma unroll
-    for (int q = 0; q < S / 2; q++) { fl[2 * q] = a[q]; fl[2 * q + 1] = b[q]; }
-  } else {
-    load_flags<S>(L.fl + base, nv, fl);
-  }
-  T my = valid ? L.cmy[j] : T(0), py = valid ? L.cpy[j] : T(0);
-  T mz = valid ? L.cmz[k] : T(0), pz = valid ? L.cpz[k] : T(0);
   SegElim<T, S> se;
+  if constexpr (SPL) {
+    const long st[4] = {-(long)L.sx, L.sx, -L.sxy, L.sxy};
+    const T ct[4] = {my, py, mz, pz};
+    if constexpr (S < 16) {
 #pragma unroll
-  for (int s = 0; s < S; s++) {
-    uint8_t f = fl[s];
-    T a = T(0), b = T(1), c = T(0), d = T(0);
-    if (s < nv) {
-      if (f & FL_BLANK) {
-        d = (f & FL_GHOST) ? eo[s] : T(0);
-      } else {
-        T amx = (f & FL_IM) ? T(0) : cmx[s], apx = (f & FL_IP) ? T(0) : cpx[s];
-        T amy = (f & FL_JM) ? T(0) : my, apy = (f & FL_JP) ? T(0) : py;
-        T amz = (f & FL_KM) ? T(0) : mz, apz = (f & FL_KP) ? T(0) : pz;
-        T diag = (-(amx + apx) + -(amy + apy)) + -(amz + apz);
-        T r = rv[s] - ejm[s] * amy - ejp[s] * apy - ekm[s] * amz - ekp[s] * apz;
-        if (tabs(diag) < T(1.0e-12)) {
-          d = eo[s];
-        } else {
-          a = amx; b = diag; c = apx; d = r;
-        }
+      for (int t = 0; t < 4; t++) {
+        T v[S];
+        ld(e + base + st[t], v);
+#pragma unroll
+        for (int q = 0; q < S; q++) rv[q] = rv[q] - v[q] * ct[t];
       }
+    } else {
+      // few wavefronts fit: all four neighbour lines in flight at once
+      // (512x512x384: 182 us against 190)
+      T v[4][S];
+#pragma unroll
+      for (int t = 0; t < 4; t++) ld(e + base + st[t], v[t]);
+#pragma unroll
+      for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int q = 0; q < S; q++) asm volatile("" : "+v"(v[t][q]));
+#pragma unroll
+      for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int q = 0; q < S; q++) rv[q] = rv[q] - v[t][q] * ct[t];
     }
-    se.push(s, a, b, c, d);
+    load_chunk<T, S>(L.cmx + i0, S, cmx);
+    load_chunk<T, S>(L.cpx + i0, S, cpx);
+    uint8_t a[S / 2], b[S / 2];
+    load_flags<S / 2>(L.fl + base, S / 2, a);
+    load_flags<S / 2>(L.fl + base + hp, S / 2, b);
+    const T dy = -(my + py), dz = -(mz + pz);
+#pragma unroll
+    for (int s = 0; s < S; s++) {
+      const uint8_t f = s < nv ? ((s & 1) ? b[s / 2] : a[s / 2]) : (uint8_t)FL_BLANK;
+      const bool fluid = !(f & FL_BLANK);
+      const T diag = (-(cmx[s] + cpx[s]) + dy) + dz;
+      se.push(s, fluid ? cmx[s] : T(0), fluid ? diag : T(1), fluid ? cpx[s] : T(0),
+              fluid ? rv[s] : ((f & FL_GHOST) ? eo[s] : T(0)));
+    }
+  } else {
+    T ejm[S], ejp[S], ekm[S], ekp[S];
+    ld(e + base - L.sx, ejm);
+    ld(e + base + L.sx, ejp);
+    ld(e + base - L.sxy, ekm);
+    ld(e + base + L.sxy, ekp);
+    load_chunk<T, S>(L.cmx + i0, nv, cmx);
+    load_chunk<T, S>(L.cpx + i0, nv, cpx);
+    load_flags<S>(L.fl + base, nv, fl);
+#pragma unroll
+    for (int s = 0; s < S; s++) {
+      const uint8_t f = s < nv ? fl[s] : (uint8_t)FL_BLANK;
+      const T amx = (f & FL_IM) ? T(0) : cmx[s], apx = (f & FL_IP) ? T(0) : cpx[s];
+      const T amy = (f & FL_JM) ? T(0) : my, apy = (f & FL_JP) ? T(0) : py;
+      const T amz = (f & FL_KM) ? T(0) : mz, apz = (f & FL_KP) ? T(0) : pz;
+      const T diag = (-(amx + apx) + -(amy + apy)) + -(amz + apz);
+      const T r = rv[s] - ejm[s] * amy - ejp[s] * apy - ekm[s] * amz - ekp[s] * apz;
+      // blank rows hold the ghost value; a fluid row with every face closed
+      // keeps its value
+      const bool fluid = !(f & FL_BLANK), row = fluid && !(tabs(diag) < T(1.0e-12));
+      se.push(s, row ? amx : T(0), row ? diag : T(1), row ? apx : T(0),
+              row ? r : ((fluid || (f & FL_GHOST)) ? eo[s] : T(0)));
+    }
   }
   se.template solve<G>();
 #pragma unroll
   for (int s = 0; s < S; s++) eo[s] = (T(1) - omega) * eo[s] + omega * se.dp[s];
+  const int ns = valid ? nv : 0;
   if constexpr (SPL) {
     T a[S / 2], b[S / 2];
 #pragma unroll
     for (int q = 0; q < S / 2; q++) { a[q] = eo[2 * q]; b[q] = eo[2 * q + 1]; }
-    store_chunk<T, S / 2>(e + base, (nv + 1) >> 1, a);
-    store_chunk<T, S / 2>(e + base + hp, nv >> 1, b);
+    store_chunk<T, S / 2>(e + base, (ns + 1) >> 1, a);
+    store_chunk<T, S / 2>(e + base + hp, ns >> 1, b);
   } else {
-    store_chunk<T, S>(e + base, nv, eo);
+    store_chunk<T, S>(e + base, ns, eo);
   }
 }
 
 // Reduced system of a line split into P segments held by the P threads
 // (tx, 0..P-1) of a block column: back recurrences of each segment, then
 // parallel cyclic reduction of the P equations (unknown = a segment's last
-// cell) with one equation per thread, double-buffered in LDS
-// [buf][seg][field][tx] (8*P*blockDim.x elements).  Every thread of the
-// block must call it (it synchronises the block).  Returns the unknowns of
-// the previous segment (XL, 0 for the first) and of this segment (XS).
+// cell) with one equation per thread, double-buffered in LDS as one vector
+// (A, B, C, R) per equation; row P of each buffer holds the identity equation
+// read past the ends of a line (2 (P + 1) blockDim.x vectors).  Every thread
+// of the block must call it (it synchronises the block).  Returns the
+// unknowns of the previous segment (XL, 0 for the first) and of this segment
+// (XS).
+template <typename T>
+struct alignas(4 * sizeof(T)) RedEq {
+  T a, b, c, r;
+};
 template <typename T, int LS>
-__device__ inline void seg_reduced_solve(T *sh, int P, int tx, int seg, SegElim<T, LS> &se, T &XL, T &XS) {
+__device__ inline void seg_reduced_solve(RedEq<T> *sh, int P, int tx, int seg, SegElim<T, LS> &se, T &XL, T &XS) {
   T cl, dl, fl;
   se.back(cl, dl, fl);
   const int TXb = blockDim.x;
-  T *bufA = sh, *bufB = sh + 4 * TXb * P;
-  auto E_ = [&](T *buf, int s, int fld) -> T & { return buf[((long)s * 4 + fld) * TXb + tx]; };
-  E_(bufB, seg, 0) = se.dp[0]; E_(bufB, seg, 1) = se.fp[0]; E_(bufB, seg, 2) = se.cp[0];
+  RedEq<T> *cur = sh, *nxt = sh + (P + 1) * TXb;
+  if (seg == 0) cur[P * TXb + tx] = nxt[P * TXb + tx] = RedEq<T>{T(0), T(1), T(0), T(0)};
+  nxt[seg * TXb + tx] = RedEq<T>{se.fp[0], se.cp[0], se.dp[0], T(0)};
   __syncthreads();
   T D0n = T(0), F0n = T(0), G0n = T(0);
-  if (seg + 1 < P) { D0n = E_(bufB, seg + 1, 0); F0n = E_(bufB, seg + 1, 1); G0n = E_(bufB, seg + 1, 2); }
+  if (seg + 1 < P) {
+    const RedEq<T> v = nxt[(seg + 1) * TXb + tx];
+    F0n = v.a; G0n = v.b; D0n = v.c;
+  }
   T A = -fl, B = T(1) + cl * F0n, C = cl * G0n, R = dl - cl * D0n;
-  T *cur = bufA, *nxt = bufB;
-  E_(cur, seg, 0) = A; E_(cur, seg, 1) = B; E_(cur, seg, 2) = C; E_(cur, seg, 3) = R;
+  cur[seg * TXb + tx] = RedEq<T>{A, B, C, R};
   __syncthreads();
   for (int d = 1; d < P; d <<= 1) {
-    T Am = T(0), Bm = T(1), Cm = T(0), Rm = T(0), Ap = T(0), Bp = T(1), Cp = T(0), Rp = T(0);
-    if (seg - d >= 0) {
-      Am = E_(cur, seg - d, 0); Bm = E_(cur, seg - d, 1); Cm = E_(cur, seg - d, 2); Rm = E_(cur, seg - d, 3);
-    }
-    if (seg + d < P) {
-      Ap = E_(cur, seg + d, 0); Bp = E_(cur, seg + d, 1); Cp = E_(cur, seg + d, 2); Rp = E_(cur, seg + d, 3);
-    }
-    T k1 = A * fast_rcp(Bm), k2 = C * fast_rcp(Bp);
-    T nA = -Am * k1, nC = -Cp * k2;
-    T nB = B - Cm * k1 - Ap * k2, nR = R - Rm * k1 - Rp * k2;
-    A = nA; B = nB; C = nC; R = nR;
-    E_(nxt, seg, 0) = A; E_(nxt, seg, 1) = B; E_(nxt, seg, 2) = C; E_(nxt, seg, 3) = R;
+    const RedEq<T> m = cur[(seg >= d ? seg - d : P) * TXb + tx];
+    const RedEq<T> p = cur[(seg + d < P ? seg + d : P) * TXb + tx];
+    const T k1 = A * fast_rcp(m.b), k2 = C * fast_rcp(p.b);
+    A = -m.a * k1;
+    B = B - m.c * k1 - p.a * k2;
+    C = -p.c * k2;
+    R = R - m.r * k1 - p.r * k2;
+    nxt[seg * TXb + tx] = RedEq<T>{A, B, C, R};
     __syncthreads();
-    T *t = cur; cur = nxt; nxt = t;
+    RedEq<T> *t = cur; cur = nxt; nxt = t;
   }
   XS = R * fast_rcp(B);
-  E_(nxt, seg, 0) = XS;
+  T *xs = reinterpret_cast<T *>(nxt);
+  xs[seg * TXb + tx] = XS;
   __syncthreads();
-  XL = seg > 0 ? E_(nxt, seg - 1, 0) : T(0);
+  XL = seg > 0 ? xs[(seg - 1) * TXb + tx] : T(0);
 }
 
 // ---------------------------------------------------------------------
@@ -1696,214 +1734,120 @@ __device__ inline void seg_reduced_solve(T *sh, int P, int tx, int seg, SegElim<
 // (i, plane) with (i + plane) % 2 == colour, plane = k for DIR = 1 (lines
 // along j) and plane = j for DIR = 2 (lines along k), so every neighbour
 // line of a line has the other colour and the pass is deterministic.  A
-// block of TX x P threads covers TX lines of one colour (every other i of
-// a 2*TX-wide tile) and P segments of LS cells of each line.  Each thread
-// eliminates its segment in registers, the P reduced equations of a line
-// are solved by parallel cyclic reduction in LDS (one equation per thread),
-// and every thread back-substitutes.  The tile's loads cover 2*TX consecutive i, half of
-// them own cells and half the neighbour lines read by the stencil.
+// block of TX x P threads covers TX lines of one colour and P segments of LS
+// cells of each line.  Each thread eliminates its segment in registers, the
+// P reduced equations of a line are solved by parallel cyclic reduction in
+// LDS (one equation per thread), and every thread back-substitutes.
+//
+// SPL: the finest level's colour-split rows (sidx, half-row offset hp): a
+// colour's cells are contiguous half rows, their x-neighbours the other
+// half, and its faces are closed on the outer boundary only, where the
+// coefficients are 0, so its rows test the blank flag alone.  Else the
+// natural rows with the level's closed faces, own cells and neighbour lines
+// interleaved.
+//
+// The cells are read PF ahead of their elimination.  The results of a row
+// are pinned before the next loads: left alone the compiler reads the whole
+// segment first, and the registers that takes cost more blocks per CU than
+// the extra loads in flight are worth (six wavefronts per SIMD hold three
+// 512-thread blocks of 12-cell segments: 83 registers instead of 80 cost
+// 11%).  Rows are chosen by selects.  One
+// colour pass on the split level, FP32: 256x192x192 15.6 us in y, 16.0 in z
+// (LS = 12, PF = 2, 32-line tiles) against 20.6 and 20.8 with a branch per
+// flag, LS = 8 and cells four ahead; 384x256x256 42 and 43 (LS = 16, PF = 4)
+// against 65 and 67; FP64 256x192x192 33.6 against 57 in natural rows.
 // ---------------------------------------------------------------------
-template <typename T, int LS, int DIR, bool UPF = false>
-__global__ void __launch_bounds__(1024) k_yzline(LevelArgs<T> Lv, const T *__restrict__ rhs, T *__restrict__ e,
-                                                 int color, T omega) {
+template <typename T, int LS>
+constexpr int yz_prefetch() { return LS <= 4 ? LS : (LS == 8 ? 4 : (LS == 16 && sizeof(T) == 4 ? 4 : 2)); }
+template <typename T, int LS, int DIR, bool SPL>
+__global__ void __launch_bounds__(sizeof(T) == 4 ? 1024 : 512)
+    __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 2 : (LS == 12 && SPL ? 6 : 4), 8)))
+    k_yzline(LevelArgs<T> Lv, int hp, const T *__restrict__ rhs, T *__restrict__ e, int color, T omega) {
+  constexpr int PF = yz_prefetch<T, LS>();
   extern __shared__ unsigned char smem_raw[];
-  T *sh = reinterpret_cast<T *>(smem_raw);
-  const int P = blockDim.y;
-  const int tx = threadIdx.x, seg = threadIdx.y;
-  const int lb = xcd_block(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
-  const int tile = lb % gridDim.x, plane = lb / gridDim.x;
-  const int i = 2 * (tile * blockDim.x + tx) + ((plane + color) & 1);
-  const int n = DIR == 1 ? Lv.cy : Lv.cz;
-  const bool ok = ((DIR == 1) ? (plane < Lv.cz) : (plane < Lv.cy)) && i < Lv.cx;
-  const int m0 = seg * LS;
-  // coefficients constant along the line
-  T mx = T(0), px = T(0), mo = T(0), po = T(0);
-  if (ok) {
-    mx = Lv.cmx[i]; px = Lv.cpx[i];
-    mo = DIR == 1 ? Lv.cmz[plane] : Lv.cmy[plane];
-    po = DIR == 1 ? Lv.cpz[plane] : Lv.cpy[plane];
-  }
-  const long ostride = DIR == 1 ? Lv.sxy : (long)Lv.sx;   // the other transverse direction
-  const long lstride = DIR == 1 ? (long)Lv.sx : Lv.sxy;   // along the line
-  const uint8_t FO_M = DIR == 1 ? FL_KM : FL_JM, FO_P = DIR == 1 ? FL_KP : FL_JP;
-  const uint8_t FL_M = DIR == 1 ? FL_JM : FL_KM, FL_P = DIR == 1 ? FL_JP : FL_KP;
-  const T *cml = DIR == 1 ? Lv.cmy : Lv.cmz;
-  const T *cpl = DIR == 1 ? Lv.cpy : Lv.cpz;
-  long id0 = 0;
-  if (ok) id0 = DIR == 1 ? lidx(Lv.sx, Lv.sxy, i, m0, plane) : lidx(Lv.sx, Lv.sxy, i, plane, m0);
-  // the line coefficients of this segment, loaded once ahead of the cells
-  // (wavefront-uniform scalar loads when the tile is 64 lines wide)
-  T cq_m[LS], cq_p[LS];
-  const int m0u = blockDim.x >= 64 ? __builtin_amdgcn_readfirstlane(m0) : m0;
-#pragma unroll
-  for (int m = 0; m < LS; m++) {
-    const int q = m0u + m;
-    cq_m[m] = q < n ? cml[q] : T(0);
-    cq_p[m] = q < n ? cpl[q] : T(0);
-  }
-  // UPF: all loads of the segment are issued unconditionally (cells past the
-  // line or the level read a valid cell instead and are then ignored), so
-  // that they are all in flight before the first row is built (latency-bound
-  // small levels; on large levels the extra registers cost occupancy)
-  const long idsafe = lidx(Lv.sx, Lv.sxy, 0, 0, 0);
-  constexpr int NU = UPF ? LS : 1;
-  uint8_t fv[NU];
-  T evv[NU], elv[NU], erv[NU], ezm[NU], ezp[NU], rvv[NU];
-  auto load_cell = [&](int m, int slot) {
-    const bool live = ok && m0 + m < n;
-    const long id = live ? id0 + m * lstride : idsafe;
-    fv[slot] = Lv.fl[id];
-    evv[slot] = e[id];
-    elv[slot] = e[id - 1];
-    erv[slot] = e[id + 1];
-    ezm[slot] = e[id - ostride];
-    ezp[slot] = e[id + ostride];
-    rvv[slot] = rhs[id];
-  };
-  if constexpr (UPF) {
-#pragma unroll
-    for (int m = 0; m < LS; m++) load_cell(m, m);
-  }
-  T eo[LS];
-  SegElim<T, LS> se;
-#pragma unroll
-  for (int m = 0; m < LS; m++) {
-    T a = T(0), b = T(1), c = T(0), d = T(0);
-    eo[m] = T(0);
-    int q = m0 + m;
-    const int sl = UPF ? m : 0;
-    if constexpr (!UPF) {
-      if (ok && q < n) load_cell(m, 0);
-    }
-    if (ok && q < n) {
-      uint8_t f = fv[sl];
-      T ev = evv[sl];
-      eo[m] = ev;
-      if (f & FL_BLANK) {
-        d = (f & FL_GHOST) ? ev : T(0);
-      } else {
-        T amx = (f & FL_IM) ? T(0) : mx, apx = (f & FL_IP) ? T(0) : px;
-        T amo = (f & FO_M) ? T(0) : mo, apo = (f & FO_P) ? T(0) : po;
-        T am = (f & FL_M) ? T(0) : cq_m[m], ap = (f & FL_P) ? T(0) : cq_p[m];
-        // (acx + acy + acz) in the reference's order
-        T diag = DIR == 1 ? (-(amx + apx) + -(am + ap)) + -(amo + apo) : (-(amx + apx) + -(amo + apo)) + -(am + ap);
-        T r = rvv[sl] - elv[sl] * amx - erv[sl] * apx - ezm[sl] * amo - ezp[sl] * apo;
-        if (tabs(diag) < T(1.0e-12)) {
-          d = ev;
-        } else {
-          a = am; b = diag; c = ap; d = r;
-        }
-      }
-    }
-    se.push(m, a, b, c, d);
-  }
-  T XL, XS;
-  seg_reduced_solve<T, LS>(sh, P, tx, seg, se, XL, XS);
-  if (!ok) return;
-  se.combine(XL, XS);
-#pragma unroll
-  for (int m = 0; m < LS; m++) {
-    if (m0 + m < n) e[id0 + m * lstride] = (T(1) - omega) * eo[m] + omega * se.dp[m];
-  }
-}
-
-// k_yzline on the colour-split FP32 level 0 (sidx, half-row offset hp):
-// a colour's cells are contiguous half rows, their x-neighbours the
-// other half.  The cells of a segment are read PF ahead of their
-// elimination (every load unconditional: cells past the line or the level
-// read a valid cell and are ignored), and the register budget is held at
-// six wavefronts per SIMD so that two 768-thread blocks share a CU.
-template <int LS, int DIR>
-__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(6, 8)))
-k_yzline_split(LevelArgs<float> Lv, int hp, const float *__restrict__ rhs, float *__restrict__ e, int color,
-               float omega) {
-  constexpr int PF = LS < 4 ? LS : 4;
-  extern __shared__ unsigned char smem_raw[];
-  float *sh = reinterpret_cast<float *>(smem_raw);
   const int P = blockDim.y;
   const int tx = threadIdx.x, seg = threadIdx.y;
   const int lb = xcd_block(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
   const int tile = lb % gridDim.x, plane = lb / gridDim.x;
   const int par = (plane + color) & 1;
-  const int i = 2 * (tile * blockDim.x + tx) + par;
+  const int h = tile * blockDim.x + tx;
+  const int i = 2 * h + par;
   const int n = DIR == 1 ? Lv.cy : Lv.cz;
-  const bool ok = ((DIR == 1) ? (plane < Lv.cz) : (plane < Lv.cy)) && i < Lv.cx;
+  const bool ok = i < Lv.cx;
   const int m0 = seg * LS;
-  float mx = 0.f, px = 0.f, mo = 0.f, po = 0.f;
-  if (ok) {
-    mx = Lv.cmx[i]; px = Lv.cpx[i];
-    mo = DIR == 1 ? Lv.cmz[plane] : Lv.cmy[plane];
-    po = DIR == 1 ? Lv.cpz[plane] : Lv.cpy[plane];
-  }
-  const long ostride = DIR == 1 ? Lv.sxy : (long)Lv.sx;
-  const long lstride = DIR == 1 ? (long)Lv.sx : Lv.sxy;
-  const uint8_t FO_M = DIR == 1 ? FL_KM : FL_JM, FO_P = DIR == 1 ? FL_KP : FL_JP;
-  const uint8_t FL_M = DIR == 1 ? FL_JM : FL_KM, FL_P = DIR == 1 ? FL_JP : FL_KP;
-  const float *cml = DIR == 1 ? Lv.cmy : Lv.cmz;
-  const float *cpl = DIR == 1 ? Lv.cpy : Lv.cpz;
-  const long idsafe = sidx(Lv.sx, Lv.sxy, hp, 0, 0, 0);
-  long id0 = idsafe;
-  if (ok) id0 = DIR == 1 ? sidx(Lv.sx, Lv.sxy, hp, i, m0, plane) : sidx(Lv.sx, Lv.sxy, hp, i, plane, m0);
-  // offsets of the x-neighbours i-1 and i+1 (the other half of the row)
-  const long dlo = par ? -(long)hp : (long)hp - 1;
-  const long dhi = par ? 1 - (long)hp : (long)hp;
+  const long ostride = DIR == 1 ? Lv.sxy : (long)Lv.sx;   // the other transverse direction
+  const long lstride = DIR == 1 ? (long)Lv.sx : Lv.sxy;   // along the line
+  const T *cml = DIR == 1 ? Lv.cmy : Lv.cmz;
+  const T *cpl = DIR == 1 ? Lv.cpy : Lv.cpz;
+  // uniform offset of the plane's first cell of the colour, the line's
+  // offset from it (cells past the line or the level read the line's first
+  // cell, or the plane's, instead and are ignored) and the x-neighbours'
+  const int pj = DIR == 1 ? 0 : plane, pk = DIR == 1 ? plane : 0;
+  const long base = SPL ? sidx(Lv.sx, Lv.sxy, hp, par, pj, pk) : lidx(Lv.sx, Lv.sxy, par, pj, pk);
+  const long v0 = ok ? (SPL ? h : 2 * h) : 0;
+  const long dlo = SPL ? (par ? -(long)hp : (long)hp - 1) : -1, dhi = SPL ? (par ? 1 - (long)hp : (long)hp) : 1;
+  const T *eb = e + base, *rb = rhs + base;
+  const uint8_t *fb = Lv.fl + base;
+  // coefficients constant along the line
+  const int ic = ok ? i : 0;
+  const T mx = Lv.cmx[ic], px = Lv.cpx[ic];
+  const T mo = DIR == 1 ? Lv.cmz[plane] : Lv.cmy[plane], po = DIR == 1 ? Lv.cpz[plane] : Lv.cpy[plane];
+  const T dx = -(mx + px), dox = -(mo + po);
+  constexpr uint8_t FO_M = DIR == 1 ? FL_KM : FL_JM, FO_P = DIR == 1 ? FL_KP : FL_JP;
+  constexpr uint8_t FL_M = DIR == 1 ? FL_JM : FL_KM, FL_P = DIR == 1 ? FL_JP : FL_KP;
+  T eo[LS];
   uint8_t fv[PF];
-  float evv[PF], elv[PF], erv[PF], ezm[PF], ezp[PF], rvv[PF], cqm[PF], cqp[PF];
-  auto load_cell = [&](int m, int slot) {
-    const bool live = ok && m0 + m < n;
-    const long id = live ? id0 + m * lstride : idsafe;
-    const int q = live ? m0 + m : 0;
-    fv[slot] = Lv.fl[id];
-    evv[slot] = e[id];
-    elv[slot] = e[id + dlo];
-    erv[slot] = e[id + dhi];
-    ezm[slot] = e[id - ostride];
-    ezp[slot] = e[id + ostride];
-    rvv[slot] = rhs[id];
-    cqm[slot] = cml[q];
-    cqp[slot] = cpl[q];
+  T cm[PF], cp[PF], rv[PF], el[PF], er[PF], zm[PF], zp[PF];
+  auto load_cell = [&](int m) {
+    const int s = m % PF, q = m0 + m < n ? m0 + m : 0;
+    const long o = v0 + q * lstride;
+    fv[s] = fb[o];
+    eo[m] = eb[o];
+    cm[s] = cml[q];
+    cp[s] = cpl[q];
+    rv[s] = rb[o];
+    el[s] = eb[o + dlo];
+    er[s] = eb[o + dhi];
+    zm[s] = eb[o - ostride];
+    zp[s] = eb[o + ostride];
   };
 #pragma unroll
-  for (int m = 0; m < PF; m++) load_cell(m, m);
-  float eo[LS];
-  SegElim<float, LS> se;
+  for (int m = 0; m < PF; m++) load_cell(m);
+  SegElim<T, LS> se;
 #pragma unroll
   for (int m = 0; m < LS; m++) {
-    const int sl = m % PF;
-    const uint8_t f = fv[sl];
-    const float ev = evv[sl], el = elv[sl], er = erv[sl], zm = ezm[sl], zp = ezp[sl], rv = rvv[sl];
-    const float cm = cqm[sl], cp = cqp[sl];
-    if (m + PF < LS) load_cell(m + PF, sl);
-    float a = 0.f, b = 1.f, c = 0.f, d = 0.f;
-    const bool live = ok && m0 + m < n;
-    eo[m] = live ? ev : 0.f;
-    if (live) {
-      if (f & FL_BLANK) {
-        d = (f & FL_GHOST) ? ev : 0.f;
-      } else {
-        const float amx = (f & FL_IM) ? 0.f : mx, apx = (f & FL_IP) ? 0.f : px;
-        const float amo = (f & FO_M) ? 0.f : mo, apo = (f & FO_P) ? 0.f : po;
-        const float am = (f & FL_M) ? 0.f : cm, ap = (f & FL_P) ? 0.f : cp;
-        // (acx + acy + acz) in the reference's order
-        const float diag =
-            DIR == 1 ? (-(amx + apx) + -(am + ap)) + -(amo + apo) : (-(amx + apx) + -(amo + apo)) + -(am + ap);
-        const float r = rv - el * amx - er * apx - zm * amo - zp * apo;
-        if (tabs(diag) < 1.0e-12f) {
-          d = ev;
-        } else {
-          a = am; b = diag; c = ap; d = r;
-        }
-      }
+    const int s = m % PF;
+    const uint8_t f = m0 + m < n ? fv[s] : (uint8_t)FL_BLANK;
+    const bool fluid = !(f & FL_BLANK);
+    if constexpr (SPL) {
+      const T r = rv[s] - el[s] * mx - er[s] * px - zm[s] * mo - zp[s] * po;
+      const T dl = -(cm[s] + cp[s]);
+      // (acx + acy + acz) in the reference's order
+      const T diag = DIR == 1 ? (dx + dl) + dox : (dx + dox) + dl;
+      se.push(m, fluid ? cm[s] : T(0), fluid ? diag : T(1), fluid ? cp[s] : T(0),
+              fluid ? r : ((f & FL_GHOST) ? eo[m] : T(0)));
+    } else {
+      const T amx = (f & FL_IM) ? T(0) : mx, apx = (f & FL_IP) ? T(0) : px;
+      const T amo = (f & FO_M) ? T(0) : mo, apo = (f & FO_P) ? T(0) : po;
+      const T am = (f & FL_M) ? T(0) : cm[s], ap = (f & FL_P) ? T(0) : cp[s];
+      const T diag = DIR == 1 ? (-(amx + apx) + -(am + ap)) + -(amo + apo) : (-(amx + apx) + -(amo + apo)) + -(am + ap);
+      const T r = rv[s] - el[s] * amx - er[s] * apx - zm[s] * amo - zp[s] * apo;
+      // blank rows hold the ghost value; a fluid row with every face closed
+      // keeps its value
+      const bool row = fluid && !(tabs(diag) < T(1.0e-12));
+      se.push(m, row ? am : T(0), row ? diag : T(1), row ? ap : T(0),
+              row ? r : ((fluid || (f & FL_GHOST)) ? eo[m] : T(0)));
     }
-    se.push(m, a, b, c, d);
+    if (PF < LS) asm volatile("" : "+v"(se.dp[m]), "+v"(se.cp[m]), "+v"(se.fp[m])::"memory");
+    if (m + PF < LS) load_cell(m + PF);
   }
-  float XL, XS;
-  seg_reduced_solve<float, LS>(sh, P, tx, seg, se, XL, XS);
+  T XL, XS;
+  seg_reduced_solve<T, LS>(reinterpret_cast<RedEq<T> *>(smem_raw), P, tx, seg, se, XL, XS);
   if (!ok) return;
   se.combine(XL, XS);
 #pragma unroll
   for (int m = 0; m < LS; m++) {
-    if (m0 + m < n) e[id0 + m * lstride] = (1.f - omega) * eo[m] + omega * se.dp[m];
+    if (m0 + m < n) e[base + v0 + (m0 + m) * lstride] = (T(1) - omega) * eo[m] + omega * se.dp[m];
   }
 }
 
@@ -2427,7 +2371,7 @@ __global__ void __launch_bounds__(1024) k_tdma_seg(int n, int nlines, const doub
                                                    const double *__restrict__ B, const double *__restrict__ C,
                                                    const double *__restrict__ Rr, double *__restrict__ U) {
   extern __shared__ unsigned char smem_raw[];
-  double *sh = reinterpret_cast<double *>(smem_raw);
+  RedEq<double> *sh = reinterpret_cast<RedEq<double> *>(smem_raw);
   const int P = blockDim.y;
   const int tx = threadIdx.x, seg = threadIdx.y;
   const int line = blockIdx.x * blockDim.x + tx;

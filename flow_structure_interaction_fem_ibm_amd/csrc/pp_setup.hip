@@ -97,6 +97,15 @@ static T *dev_upload(const std::vector<T> &h) {
   hipMemcpy(d, h.data(), sizeof(T) * h.size(), hipMemcpyHostToDevice);
   return d;
 }
+// Line coefficients for the device: 0 across the outer faces (closed on
+// every level) and zero-padded, so that a lane's chunk past the end of a
+// line can be read whole.
+static std::vector<double> line_coef(std::vector<double> h, bool lower) {
+  if (h.empty()) return h;
+  (lower ? h.front() : h.back()) = 0.0;
+  h.resize(h.size() + kMaxLine, 0.0);
+  return h;
+}
 template <typename T>
 static std::vector<float> to_f32(const std::vector<T> &h) {
   std::vector<float> r(h.size());
@@ -341,6 +350,16 @@ int setup_split0(pp_ctx *c) {
   int G, S;
   line_shape(L.cx, G, S, 4);
   if (!by2 || S % 2 != 0) return PP_OK;
+  // the split kernels' fluid rows have no guard against a vanishing diagonal
+  // (the row's open faces, the outer ones left out)
+  double dmin = 0.0;
+  for (int d = 0; d < 3; d++) {
+    const size_t n = L.cm[d].size();
+    double m = INFINITY;
+    for (size_t i = 0; i < n; i++) m = std::min(m, (i > 0 ? L.cm[d][i] : 0.0) + (i + 1 < n ? L.cp[d][i] : 0.0));
+    dmin += m;
+  }
+  if (!(dmin > 2.0e-12)) return PP_OK;
   sp.hp = ((L.cx / 2 + 2 + 31) / 32) * 32;
   sp.sx = SPLIT_E0 + 2 * sp.hp;
   sp.sxy = (long)sp.sx * (L.cy + 2);
@@ -423,8 +442,9 @@ int upload_levels(pp_ctx *c) {
     Level &L = c->lv[l];
     if (hipMalloc(&L.flags, L.total) != hipSuccess) L.flags = nullptr;
     for (int d = 0; d < 3; d++) {
-      L.cm64[d] = dev_upload(L.cm[d]); L.cp64[d] = dev_upload(L.cp[d]); L.w64[d] = dev_upload(L.w[d]);
-      L.cm32[d] = dev_upload(to_f32(L.cm[d])); L.cp32[d] = dev_upload(to_f32(L.cp[d]));
+      const std::vector<double> cm = line_coef(L.cm[d], true), cp = line_coef(L.cp[d], false);
+      L.cm64[d] = dev_upload(cm); L.cp64[d] = dev_upload(cp); L.w64[d] = dev_upload(L.w[d]);
+      L.cm32[d] = dev_upload(to_f32(cm)); L.cp32[d] = dev_upload(to_f32(cp));
       L.w32[d] = dev_upload(to_f32(L.w[d]));
       if (l + 1 < c->lv.size()) {
         L.wpar64[d] = dev_upload(L.wpar[d]); L.wpar32[d] = dev_upload(to_f32(L.wpar[d]));
