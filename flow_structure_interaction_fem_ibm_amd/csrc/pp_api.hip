@@ -1986,8 +1986,8 @@ int32_t pp_set_vel_ghosts(pp_ctx *c, const double *coeffD, double bi_weight, dou
   }
   HIPCHK(hipSetDevice(c->device));
   hipFree(g.v_cD); hipFree(g.v_buf[0]); hipFree(g.v_buf[1]); hipFree(g.v_kind); hipFree(g.v_off);
-  hipFree(g.v_off_s); hipFree(g.g_ref_s);
-  g.v_cD = g.v_buf[0] = g.v_buf[1] = nullptr; g.v_kind = nullptr; g.v_off = g.v_off_s = g.g_ref_s = nullptr;
+  hipFree(g.v_off_s); hipFree(g.g_ref_s); hipFree(g.v_base);
+  g.v_cD = g.v_buf[0] = g.v_buf[1] = g.v_base = nullptr; g.v_kind = nullptr; g.v_off = g.v_off_s = g.g_ref_s = nullptr;
   g.have_vel = false;
   const int n = g.n;
   std::vector<int> kind(8L * n);
@@ -2048,6 +2048,7 @@ int32_t pp_set_vel_ghosts(pp_ctx *c, const double *coeffD, double bi_weight, dou
     HIPCHK(hipMalloc(&g.v_off, sizeof(long) * 8 * n));
     HIPCHK(hipMalloc(&g.v_buf[0], sizeof(double) * 3 * n));
     HIPCHK(hipMalloc(&g.v_buf[1], sizeof(double) * 3 * n));
+    HIPCHK(hipMalloc(&g.v_base, sizeof(double) * 3 * n));
     HIPCHK(hipMemcpy(g.v_cD, cd.data(), sizeof(double) * 8 * n, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(g.v_kind, kind.data(), sizeof(int) * 8 * n, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(g.v_off, off.data(), sizeof(long) * 8 * n, hipMemcpyHostToDevice));
@@ -2067,25 +2068,30 @@ int32_t pp_set_vel_ghosts(pp_ctx *c, const double *coeffD, double bi_weight, dou
 }  // extern "C"
 
 namespace {
-// GCM_vel_set_bc_internal on device fields: gather the ghost cells'
-// (u, v, w), the Jacobi sweeps fixed by pp_set_vel_ghosts, scatter
-// (fields in the momentum solve's split rows when rw is given; the ghosts'
-// new values then go into its masked right-hand sides rw too)
+// GCM_vel_set_bc_internal on device fields: the Jacobi sweeps fixed by
+// pp_set_vel_ghosts, at least two (the first reads the ghosts' values from
+// the fields the last one writes).  Fields in the momentum solve's split
+// rows when rw is given; the ghosts' new values then go into its masked
+// right-hand sides rw too.
 void vel_ghosts(pp_ctx *c, double *d_u, double *d_v, double *d_w, const double *d_vbi, double *const *rw = nullptr) {
   GhostTables &g = c->gh;
   if (g.n == 0) return;
   hipStream_t s = c->stream;
-  dim3 gg((g.n + 255) / 256), blk(256);
+  const dim3 grid((unsigned)((8L * g.n + 255) / 256)), blk(256);
   const long *gref = rw ? g.g_ref_s : g.g_ref, *voff = rw ? g.v_off_s : g.v_off;
-  k_vel_ghost_gather<double><<<gg, blk, 0, s>>>(g.n, gref, d_u, d_v, d_w, g.v_buf[0]);
+  k_vel_ghost_first<<<grid, blk, 0, s>>>(g.n, g.v_cD, g.v_kind, voff, g.v_bw, g.v_iw, d_vbi, d_u, d_v, d_w, g.v_base,
+                                         g.v_buf[0]);
+  const int sweeps = std::max(g.v_sweeps, 2);
   int cur = 0;
-  for (int q = 0; q < g.v_sweeps; q++) {
-    k_vel_ghost_sweep<<<gg, blk, 0, s>>>(g.n, g.v_cD, g.v_kind, voff, g.v_bw, g.v_iw, d_vbi, d_u, d_v, d_w,
-                                         g.v_buf[cur], g.v_buf[1 - cur]);
+  for (int q = 1; q < sweeps; q++) {
+    VelGhostOut O{};
+    if (q + 1 == sweeps) {
+      O = VelGhostOut{gref, d_u, d_v, d_w, nullptr, nullptr, nullptr};
+      if (rw) { O.u2 = rw[0]; O.v2 = rw[1]; O.w2 = rw[2]; }
+    }
+    k_vel_ghost_next<<<grid, blk, 0, s>>>(g.n, g.v_cD, g.v_kind, g.v_iw, g.v_base, g.v_buf[cur], g.v_buf[1 - cur], O);
     cur ^= 1;
   }
-  k_vel_ghost_scatter<<<gg, blk, 0, s>>>(g.n, gref, g.v_buf[cur], d_u, d_v, d_w, rw ? rw[0] : nullptr,
-                                         rw ? rw[1] : nullptr, rw ? rw[2] : nullptr);
 }
 }  // namespace
 

@@ -146,7 +146,7 @@ struct GhostTables {
   // Dirichlet coefficients, per stencil entry the ghost index it reads
   // (>= 0), -1 for the field at v_off, -2 for the body-intercept value
   std::vector<long> h_s_raw;                    // stencil offsets, outer layer not clamped
-  double *v_cD = nullptr, *v_buf[2] = {nullptr, nullptr};
+  double *v_cD = nullptr, *v_buf[2] = {nullptr, nullptr}, *v_base = nullptr;
   int *v_kind = nullptr;
   long *v_off = nullptr;
   long *v_off_s = nullptr, *g_ref_s = nullptr;  // v_off and g_ref in the momentum solve's split rows

@@ -136,7 +136,7 @@ void free_ghosts(pp_ctx *c) {
                   g.nb_ref, g.nb_al, g.nb_w64, g.nb_w32, g.t_ref, g.t_al, g.t_ptr, g.t_ghost, g.t_coef64,
                   g.t_coef32, g.t_vinv64, g.t_vinv32, g.g_tidx, g.lam64[0], g.lam64[1], g.rhsg64,
                   g.tbase64, g.lam32[0], g.lam32[1], g.rhsg32, g.tbase32, g.olam64[0], g.olam64[1],
-                  g.orhsg64, g.otbase64, g.v_cD, g.v_buf[0], g.v_buf[1], g.v_kind, g.v_off, g.v_off_s, g.g_ref_s,
+                  g.orhsg64, g.otbase64, g.v_cD, g.v_buf[0], g.v_buf[1], g.v_kind, g.v_off, g.v_off_s, g.g_ref_s, g.v_base,
                   g.ct_ref, g.ct_al, g.ct_ptr, g.ct_ghost, g.ct_w64, g.ct_vinv64, g.ctbase64,
                   g.ct_w32, g.ct_vinv32, g.ctbase32, g.g_as, g.c_as, g.nb_as, g.ct_as};
   for (void *p : ptrs) hipFree(p);
