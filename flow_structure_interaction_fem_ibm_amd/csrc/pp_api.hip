@@ -35,7 +35,7 @@ using namespace pp;
 // ---------------------------------------------------------------------
 constexpr long kNoAllocPartials = 1L << 19;   // workgroups of the first stage
 constexpr long kNoAllocDoubles = kNoAllocPartials + 256 + 64;
-static __device__ __align__(256) double scratch[kNoAllocDoubles];
+static __device__ __align__(256) double scratch[kNoAllocDoubles];  // its last entry: the reductions' counter
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -703,23 +703,31 @@ int precondition(pp_ctx *c, const pp_solve_opts *o, pp_solve_stats &S, bool in_s
 // ---------------------------------------------------------------------
 CellLaunch ref_launch(const pp_ctx *c) { return cell_launch(c->nxc, c->nyc, c->nzc); }
 
-// two-stage reductions of per-workgroup partials (kRedStage workgroups,
-// then one): fixed order, so deterministic
-constexpr int kRedStage = 256;
-void launch_reduce_summax(pp_ctx *c, int nblk) {
-  int chunk = (nblk + kRedStage - 1) / kRedStage;
-  k_reduce_summax_stage<<<kRedStage, 256, 0, c->stream>>>(c->d_part, nblk, chunk, c->d_part2);
-  k_reduce_summax<<<1, 256, 0, c->stream>>>(c->d_part2, kRedStage, c->d_res);
+// Reductions of per-workgroup partials: one workgroup per kRedChunk of
+// them, at most kRedStage.  The results go to d_res (for later kernels) and
+// to the pinned mirror h_res + hoff, valid there after a synchronisation.
+constexpr int kRedStage = 256, kRedChunk = 512;
+struct RedShape {
+  int grid, chunk;
+};
+RedShape red_shape(int nblk) {
+  RedShape r;
+  r.grid = std::min(kRedStage, (nblk + kRedChunk - 1) / kRedChunk);
+  r.chunk = (nblk + r.grid - 1) / r.grid;
+  return r;
 }
-void launch_reduce_sums(pp_ctx *c, int nblk, int nq) {
-  int chunk = (nblk + kRedStage - 1) / kRedStage;
-  k_reduce_sums_stage<<<kRedStage, 256, 0, c->stream>>>(c->d_part, nblk, nq, chunk, c->d_part2);
-  k_reduce_sums<<<1, 256, 0, c->stream>>>(c->d_part2, kRedStage, nq, c->d_res);
+void launch_reduce_summax(pp_ctx *c, int nblk) {
+  const RedShape r = red_shape(nblk);
+  k_reduce_summax<<<r.grid, 256, 0, c->stream>>>(c->d_part, nblk, r.chunk, c->d_part2, c->d_redcount, c->d_res, c->h_res);
+}
+void launch_reduce_sums(pp_ctx *c, int nblk, int nq, int hoff = 0, const RedScale *s2 = nullptr) {
+  const RedShape r = red_shape(nblk);
+  k_reduce_sums<<<r.grid, 256, 0, c->stream>>>(c->d_part, nblk, nq, r.chunk, c->d_part2, c->d_redcount, c->d_res,
+                                               c->h_res + hoff, s2 ? *s2 : RedScale{}, s2 ? c->d_kcoef : nullptr);
 }
 
 int reduce_summax(pp_ctx *c, int nblk) {
   launch_reduce_summax(c, nblk);
-  HIPCHK(hipMemcpyAsync(c->h_res, c->d_res, 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
   return PP_OK;
 }
@@ -789,7 +797,6 @@ int mean_remove_ref(pp_ctx *c, double *p, double *mean_out, bool fresh = true) {
     k_fresh_fill<<<cl.grid, cl.block, 0, c->stream>>>(c->ref, c->d_iblank_ref, c->d_fresh, c->d_tmp, p);
   }
   if (mean_out) {
-    HIPCHK(hipMemcpyAsync(c->h_res, c->d_res, 5 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     *mean_out = c->h_res[3] / c->h_res[4];
   }
@@ -842,7 +849,6 @@ int ensure_krylov_level(pp_ctx *c, int m) {
 // sum of nq per-block partials -> c->h_res[0..nq)
 int reduce_sums_host(pp_ctx *c, int nq, int nblk = -1) {
   launch_reduce_sums(c, nblk >= 0 ? nblk : c->nblk_red, nq);
-  HIPCHK(hipMemcpyAsync(c->h_res, c->d_res, sizeof(double) * nq, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
   return PP_OK;
 }
@@ -871,6 +877,7 @@ int reduce_sums_host(pp_ctx *c, int nq, int nblk = -1) {
 // reduced by Givens rotations on the host.  Stops at m steps, at the
 // iteration limit or when the least-squares residual meets the tolerance.
 // ---------------------------------------------------------------------
+constexpr int kResDots = 16;  // offset of a step's dots in h_res
 template <typename Ops>
 int gmres_cycle(pp_ctx *c, const pp_solve_opts *o, Ops &ops, double beta, double bden, int &outer,
                 pp_solve_stats &S) {
@@ -887,16 +894,16 @@ int gmres_cycle(pp_ctx *c, const pp_solve_opts *o, Ops &ops, double beta, double
     V.n = j + 1;
     for (int q = 0; q <= j; q++) V.u[q] = ops.u(q);
     ops.apply(j, V);
-    rc = reduce_sums_host(c, j + 1, ops.blocks());
-    if (rc) return rc;
-    for (int q = 0; q <= j; q++) {
-      double d = c->h_res[q];
-      h(q, j) = sig[j] * sig[q] * d;
-      V.c[q] = sig[q] * sig[q] * d;
-    }
+    // the dots stay on the device for the orthogonalisation (scaled to its
+    // coefficients); the host waits once per step, for them and the norm
+    RedScale s2{};
+    for (int q = 0; q <= j; q++) s2.c[q] = sig[q] * sig[q];
+    launch_reduce_sums(c, ops.blocks(), j + 1, kResDots, &s2);
+    V.cd = c->d_kcoef;
     ops.orth(j, V);
     rc = reduce_sums_host(c, 1, ops.blocks());
     if (rc) return rc;
+    for (int q = 0; q <= j; q++) h(q, j) = sig[j] * sig[q] * c->h_res[kResDots + q];
     double hn = std::sqrt(c->h_res[0]);
     h(j + 1, j) = sig[j] * hn;
     sig[j + 1] = hn > 0.0 ? 1.0 / hn : 0.0;
@@ -1116,7 +1123,6 @@ int solve_impl(pp_ctx *c, double *p, const double *rhs, const double *bc_src, co
   // compatibility projection: b_f -= (w.b + wg.bnd) / sum_f w
   if (o->project_rhs) {
     fluid_sums(c, c->d_w, c->d_b, nullptr);
-    HIPCHK(hipMemcpyAsync(c->h_res, c->d_res, 5 * sizeof(double), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
     double num = c->h_res[0], den = c->h_res[1];
     if (have_bnd) {
@@ -1130,13 +1136,9 @@ int solve_impl(pp_ctx *c, double *p, const double *rhs, const double *bc_src, co
     }
     double shift = num / den;
     S.rhs_shift = shift;
-    c->h_res[0] = shift;
-    c->h_res[1] = 1.0;
-    HIPCHK(hipMemcpyAsync(c->d_res + 8, c->h_res, 2 * sizeof(double), hipMemcpyHostToDevice, s));
-    k_fluid_shift<<<cl.grid, cl.block, 0, s>>>(c->ref, a0, c->d_b, c->d_res + 8, c->d_res + 9, -1.0);
+    k_fluid_shift<<<cl.grid, cl.block, 0, s>>>(c->ref, a0, c->d_b, -shift);
   }
   fluid_sums(c, nullptr, c->d_b, nullptr);
-  HIPCHK(hipMemcpyAsync(c->h_res, c->d_res, 5 * sizeof(double), hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
   double bnorm = std::sqrt(c->h_res[2]);
   S.b_l2 = bnorm;
@@ -1730,7 +1732,10 @@ int32_t pp_create(pp_ctx **out, const pp_grid_desc *g) {
   HIPCHK(hipMalloc(&c->d_part, sizeof(double) * (KRY_MAX + 1) * (size_t)c->nblk_red + 64));
   HIPCHK(hipMalloc(&c->d_part2, sizeof(double) * (KRY_MAX + 1) * kRedStage));
   HIPCHK(hipMalloc(&c->d_res, sizeof(double) * 32));
-  HIPCHK(hipHostMalloc(&c->h_res, sizeof(double) * 32));
+  HIPCHK(hipMalloc(&c->d_kcoef, sizeof(double) * (KRY_MAX + 1)));
+  HIPCHK(hipMalloc(&c->d_redcount, sizeof(unsigned)));
+  HIPCHK(hipMemset(c->d_redcount, 0, sizeof(unsigned)));
+  HIPCHK(hipHostMalloc(&c->h_res, sizeof(double) * 64));
   *out = c;
   return PP_OK;
 }
@@ -1747,7 +1752,7 @@ int32_t pp_destroy(pp_ctx *c) {
   hipFree(c->adw.buf);
   hipFree(c->d_nshape32); hipFree(c->d_nshape64);
   free_fresh_rows(c);
-  hipFree(c->d_part); hipFree(c->d_part2); hipFree(c->d_res);
+  hipFree(c->d_part); hipFree(c->d_part2); hipFree(c->d_res); hipFree(c->d_kcoef); hipFree(c->d_redcount);
   for (double *q : c->d_kry) hipFree(q);
   for (float *q : c->d_kryl) hipFree(q);
   for (int d = 0; d < 3; d++) {
@@ -2490,6 +2495,24 @@ int32_t pp_tdma_batched(pp_ctx *c, const double *a, const double *b, const doubl
   return PP_OK;
 }
 
+}  // extern "C"
+
+namespace {
+// k_divergence (no more blocks than nblk_red, which counts single rows);
+// returns its number of blocks
+constexpr int kDivRows = 4;
+int divergence_launch(pp_ctx *c, const double *fu, const double *fv, const double *fw, double dtinv, double *out,
+                      double *part, unsigned *counter) {
+  const CellLaunch cl = cell_launch(c->nxc, (c->nyc + kDivRows - 1) / kDivRows, c->nzc);
+  k_divergence<256, kDivRows><<<cl.grid, cl.block, 0, c->stream>>>(
+      c->ref, c->d_rdx[0], c->d_rdx[1], c->d_rdx[2], c->d_rdxinv[0], c->d_rdxinv[1], c->d_rdxinv[2], c->d_iblank_ref,
+      fu, fv, fw, dtinv, out, part, counter);
+  return (int)((long)cl.grid.x * cl.grid.y * cl.grid.z);
+}
+}  // namespace
+
+extern "C" {
+
 int32_t pp_divergence_noalloc(pp_ctx *c, const double *d_fu, const double *d_fv, const double *d_fw, double dtinv,
                               double *d_nlu0, double *sum) {
   if (!c || !d_fu || !d_fv || !d_fw || !d_nlu0) { set_error("pp_divergence_noalloc: null argument"); return PP_BAD_ARG; }
@@ -2504,19 +2527,13 @@ int32_t pp_divergence_noalloc(pp_ctx *c, const double *d_fu, const double *d_fv,
   if (!ptr) { set_error("pp_divergence_noalloc: no scratch address for device %d", c->device); return PP_HIP_ERROR; }
   double *part = ptr, *part2 = ptr + kNoAllocPartials, *res = ptr + kNoAllocPartials + 256;
   hipStream_t s = c->stream;
-  // the output's outer layer and blank cells are 0, as pp_divergence leaves
-  // them (a fill kernel, not a memset, so the call can be captured)
-  k_fill<double><<<(unsigned)((c->nref + 255) / 256), 256, 0, s>>>(d_nlu0, c->nref, 0.0);
-  CellLaunch cl = ref_launch(c);
-  k_divergence<256><<<cl.grid, cl.block, 0, s>>>(c->ref, c->d_rdx[0], c->d_rdx[1], c->d_rdx[2], c->d_rdxinv[0],
-                                                 c->d_rdxinv[1], c->d_rdxinv[2], c->d_iblank_ref, d_fu, d_fv, d_fw,
-                                                 dtinv, d_nlu0, part);
-  const int nblk = c->nblk_red, chunk = (nblk + kRedStage - 1) / kRedStage;
-  k_reduce_sums_stage<<<kRedStage, 256, 0, s>>>(part, nblk, 1, chunk, part2);
-  k_reduce_sums<<<1, 256, 0, s>>>(part2, kRedStage, 1, res);
+  unsigned *counter = reinterpret_cast<unsigned *>(res + 63);
+  const int nblk = divergence_launch(c, d_fu, d_fv, d_fw, dtinv, d_nlu0, part, counter);
+  const RedShape r = red_shape(nblk);
+  k_reduce_sums<<<r.grid, 256, 0, s>>>(part, nblk, 1, r.chunk, part2, counter, res,
+                                       sum ? c->h_res : res + 8, RedScale{}, nullptr);
   HIPCHK(hipGetLastError());
   if (sum) {
-    HIPCHK(hipMemcpyAsync(c->h_res, res, sizeof(double), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
     *sum = c->h_res[0];
   }
@@ -2536,14 +2553,7 @@ int32_t pp_divergence(pp_ctx *c, const double *fu, const double *fv, const doubl
     if (hipMalloc(&d[q], nb) != hipSuccess) { set_error("pp_divergence: hipMalloc failed"); rc = PP_HIP_ERROR; }
   if (rc == PP_OK) {
     for (int q = 0; q < 3; q++) hipMemcpyAsync(d[q], src[q], nb, hipMemcpyHostToDevice, c->stream);
-    hipMemsetAsync(d[3], 0, nb, c->stream);
-    CellLaunch cl = ref_launch(c);
-    k_divergence<256><<<cl.grid, cl.block, 0, c->stream>>>(c->ref, c->d_rdx[0], c->d_rdx[1], c->d_rdx[2],
-                                                           c->d_rdxinv[0], c->d_rdxinv[1], c->d_rdxinv[2],
-                                                           c->d_iblank_ref, d[0], d[1], d[2], dtinv, d[3],
-                                                           c->d_part);
-    launch_reduce_sums(c, c->nblk_red, 1);
-    hipMemcpyAsync(c->h_res, c->d_res, sizeof(double), hipMemcpyDeviceToHost, c->stream);
+    launch_reduce_sums(c, divergence_launch(c, d[0], d[1], d[2], dtinv, d[3], c->d_part, c->d_redcount), 1);
     hipMemcpyAsync(nlu0, d[3], nb, hipMemcpyDeviceToHost, c->stream);
     hipError_t e = hipStreamSynchronize(c->stream);
     if (e == hipSuccess) e = hipGetLastError();

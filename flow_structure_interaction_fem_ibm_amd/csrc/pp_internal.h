@@ -220,7 +220,9 @@ struct pp_ctx {
   unsigned long long *d_count = nullptr;  // set-up counter (ghost cells of the iblank)
   // reductions
   double *d_part = nullptr;            // partial sums
-  double *d_part2 = nullptr;           // first-stage results of the two-stage reductions
+  double *d_part2 = nullptr;           // first-stage results of the reductions
+  unsigned *d_redcount = nullptr;      // their workgroup counter (0 between launches)
+  double *d_kcoef = nullptr;           // Gram-Schmidt coefficients of the current Krylov step
   double *d_res = nullptr;             // final reduction results
   double *h_res = nullptr;             // pinned host mirror
   int nblk_red = 0;

@@ -182,64 +182,54 @@ __device__ inline SumMax block_summax(SumMax v) {
   return v;  // valid in thread 0
 }
 
-// partial[blk*3 + {0,1,2}] = {sum, max, arg}
-__global__ void k_reduce_summax(const double *__restrict__ part, int nblk, double *__restrict__ out) {
+// ---------------------------------------------------------------------
+// Reductions of per-workgroup partials in one launch: every workgroup
+// combines a chunk of them and the last one to finish combines the chunks'
+// results (fixed order in both stages: deterministic), writes them to out and
+// to the host's pinned mirror hout, and resets the counter.  A separate
+// second launch and a copy to the host took 5 and 4 us more per reduction,
+// twice per Krylov iteration.
+// ---------------------------------------------------------------------
+// true in every thread of the workgroup that arrives last (after the others'
+// results are visible to it)
+__device__ inline bool last_block(unsigned *counter) {
+  __shared__ bool last;
+  if (gridDim.x == 1) return true;
+  __threadfence();
+  __syncthreads();
+  if (threadIdx.x == 0) last = atomicAdd(counter, 1u) == gridDim.x - 1;
+  __syncthreads();
+  if (last) __threadfence();
+  return last;
+}
+
+// part[3*b + {0,1,2}] = {sum, max, arg}, combined into out and hout; 256 threads
+__global__ void __launch_bounds__(256) k_reduce_summax(const double *__restrict__ part, int nblk, int chunk,
+                                                       double *part2, unsigned *counter, double *__restrict__ out,
+                                                       double *__restrict__ hout) {
   SumMax v{0.0, -1.0, -1};
-  for (int b = threadIdx.x; b < nblk; b += 256) {
-    SumMax o{part[3 * b], part[3 * b + 1], (long)part[3 * b + 2]};
-    v = summax_combine(v, o);
-  }
-  // per-thread partials combined in thread order -> deterministic
+  const int b0 = blockIdx.x * chunk, b1 = min(nblk, b0 + chunk);
+  for (int b = b0 + threadIdx.x; b < b1; b += 256)
+    v = summax_combine(v, SumMax{part[3L * b], part[3L * b + 1], (long)part[3L * b + 2]});
   v = block_summax<256>(v);
-  if (threadIdx.x == 0) { out[0] = v.sum; out[1] = v.mx; out[2] = (double)v.arg; }
-}
-
-// first stage of a two-stage reduction of partials: workgroup b combines
-// partials [b*chunk, (b+1)*chunk) into out[3*b..3*b+2]
-__global__ void k_reduce_summax_stage(const double *__restrict__ part, int nblk, int chunk, double *__restrict__ out) {
-  SumMax v{0.0, -1.0, -1};
-  int b0 = blockIdx.x * chunk, b1 = min(nblk, b0 + chunk);
-  for (int b = b0 + threadIdx.x; b < b1; b += 256) {
-    SumMax o{part[3 * b], part[3 * b + 1], (long)part[3 * b + 2]};
-    v = summax_combine(v, o);
-  }
-  v = block_summax<256>(v);
-  if (threadIdx.x == 0) { out[3 * blockIdx.x] = v.sum; out[3 * blockIdx.x + 1] = v.mx; out[3 * blockIdx.x + 2] = (double)v.arg; }
-}
-
-// first stage for nq independent sums: out[b*nq + q]
-__global__ void k_reduce_sums_stage(const double *__restrict__ part, int nblk, int nq, int chunk,
-                                    double *__restrict__ out) {
-  __shared__ double s[256];
-  int b0 = blockIdx.x * chunk, b1 = min(nblk, b0 + chunk);
-  for (int q = 0; q < nq; q++) {
-    double v = 0.0;
-    for (int b = b0 + threadIdx.x; b < b1; b += 256) v += part[(long)b * nq + q];
-    s[threadIdx.x] = v;
-    __syncthreads();
-    for (int d = 128; d >= 1; d >>= 1) {
-      if (threadIdx.x < d) s[threadIdx.x] += s[threadIdx.x + d];
-      __syncthreads();
+  if (gridDim.x > 1) {
+    if (threadIdx.x == 0) {
+      part2[3 * blockIdx.x] = v.sum;
+      part2[3 * blockIdx.x + 1] = v.mx;
+      part2[3 * blockIdx.x + 2] = (double)v.arg;
     }
-    if (threadIdx.x == 0) out[(long)blockIdx.x * nq + q] = s[0];
+    if (!last_block(counter)) return;
+    v = SumMax{0.0, -1.0, -1};
+    const int b = threadIdx.x;
+    if (b < (int)gridDim.x) v = SumMax{part2[3 * b], part2[3 * b + 1], (long)part2[3 * b + 2]};
     __syncthreads();
+    v = block_summax<256>(v);
+    if (threadIdx.x == 0) *counter = 0;
   }
-}
-
-// multiple independent sums: part[blk*nq + q]
-__global__ void k_reduce_sums(const double *__restrict__ part, int nblk, int nq, double *__restrict__ out) {
-  __shared__ double s[256];
-  for (int q = 0; q < nq; q++) {
-    double v = 0.0;
-    for (int b = threadIdx.x; b < nblk; b += 256) v += part[(long)b * nq + q];
-    s[threadIdx.x] = v;
-    __syncthreads();
-    for (int d = 128; d >= 1; d >>= 1) {
-      if (threadIdx.x < d) s[threadIdx.x] += s[threadIdx.x + d];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) out[q] = s[0];
-    __syncthreads();
+  if (threadIdx.x == 0) {
+    out[0] = hout[0] = v.sum;
+    out[1] = hout[1] = v.mx;
+    out[2] = hout[2] = (double)v.arg;
   }
 }
 
@@ -365,31 +355,70 @@ __global__ void __launch_bounds__(NT) k_ref_residual(RefArgs R, LevelArgs<double
 // rhs_poisson, non-cut-cell branch (CORE_POISSON.F90:281-288), reference
 // layout, same operation order as the reference: nlu0 = dtinv*((u_{i+1}-u_i)
 // dxinv + (v_{j+1}-v_j) dyinv + (w_{k+1}-w_k) dzinv)*(1-iblank); per-block
-// partial sums of nlu0*dx*dy*dz at part[blk]
-template <int NT>
+// partial sums of nlu0*dx*dy*dz at part[blk].  ROWS rows of one plane per
+// thread, whose loads are in flight together; the cells at the edge of the
+// box write the zeros of the outer layers beside them, so that no fill runs
+// ahead of the pass.  Bound by its 4.1 arrays (307 MB at 256x192x192: 57 us
+// at the rate of a copy): 65 us, one row per thread after a fill of the output
+// 69 + 14; over the flat index, with its divisions, 89.  Also clears the
+// counter of the reduction that follows.
+template <int NT, int ROWS>
 __global__ void __launch_bounds__(NT) k_divergence(RefArgs R, const double *__restrict__ dx, const double *__restrict__ dy,
                                                    const double *__restrict__ dz, const double *__restrict__ dxinv,
                                                    const double *__restrict__ dyinv, const double *__restrict__ dzinv,
                                                    const int8_t *__restrict__ ib, const double *__restrict__ fu,
                                                    const double *__restrict__ fv, const double *__restrict__ fw,
-                                                   double dtinv, double *__restrict__ out, double *__restrict__ part) {
+                                                   double dtinv, double *__restrict__ out, double *__restrict__ part,
+                                                   unsigned *__restrict__ counter) {
 #pragma clang fp contract(off)
   __shared__ double s[NT / 64];
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  int j = blockIdx.y * blockDim.y + threadIdx.y, k = blockIdx.z;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int j0 = (blockIdx.y * blockDim.y + threadIdx.y) * ROWS, k = blockIdx.z;
   double vol = 0.0;
-  if (i < R.nxc && j < R.nyc) {
-    long id = ridx(R, i, j, k);
-    int I = i + 1, J = j + 1, K = k + 1;
-    double v = dtinv * ((fu[id + 1] - fu[id]) * dxinv[I] + (fv[id + R.ex] - fv[id]) * dyinv[J] +
-                        (fw[id + R.exy] - fw[id]) * dzinv[K]);
-    v = v * (double)(1 - ib[id]);
-    out[id] = v;
-    vol = v * dx[I] * dy[J] * dz[K];
+  if (i < R.nxc && j0 < R.nyc) {
+    const long id0 = ridx(R, i, j0, k);
+    const int I = i + 1, K = k + 1;
+    const double dxi = dxinv[I], dzi = dzinv[K], dxI = dx[I], dzK = dz[K];
+    double u0[ROWS], u1[ROWS], v0[ROWS + 1], w0[ROWS], w1[ROWS];
+    int8_t m[ROWS];
+    v0[0] = fv[id0];
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+      if (j0 + r >= R.nyc) break;
+      const long id = id0 + (long)r * R.ex;
+      u0[r] = fu[id];
+      u1[r] = fu[id + 1];
+      v0[r + 1] = fv[id + R.ex];
+      w0[r] = fw[id];
+      w1[r] = fw[id + R.exy];
+      m[r] = ib[id];
+    }
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+      const int j = j0 + r;
+      if (j >= R.nyc) break;
+      const long id = id0 + (long)r * R.ex;
+      double v = dtinv * ((u1[r] - u0[r]) * dxi + (v0[r + 1] - v0[r]) * dyinv[j + 1] + (w1[r] - w0[r]) * dzi);
+      v = v * (double)(1 - m[r]);
+      out[id] = v;
+      vol += v * dxI * dy[j + 1] * dzK;
+      // one layer in front of the cells, two behind them
+      const int a0 = i == 0 ? -1 : 0, a1 = i == R.nxc - 1 ? 2 : 0, b0 = j == 0 ? -1 : 0, b1 = j == R.nyc - 1 ? 2 : 0,
+                c0 = k == 0 ? -1 : 0, c1 = k == R.nzc - 1 ? 2 : 0;
+      if ((a0 | b0 | c0) || (a1 | b1 | c1)) {
+        for (int c = c0; c <= c1; c++)
+          for (int b = b0; b <= b1; b++)
+            for (int a = a0; a <= a1; a++)
+              if (a | b | c) out[id + a + b * (long)R.ex + c * (long)R.exy] = 0.0;
+      }
+    }
   }
-  double t = block_sum<NT>(vol, s);
-  long blk = blockIdx.x + (long)gridDim.x * (blockIdx.y + (long)gridDim.y * blockIdx.z);
-  if (threadIdx.x == 0 && threadIdx.y == 0) part[blk] = t;
+  const double t = block_sum<NT>(vol, s);
+  const long blk = blockIdx.x + (long)gridDim.x * (blockIdx.y + (long)gridDim.y * blockIdx.z);
+  if (threadIdx.x == 0 && threadIdx.y == 0) {
+    part[blk] = t;
+    if (blk == 0) *counter = 0;
+  }
 }
 
 // ---------------------------------------------------------------------
@@ -869,17 +898,16 @@ __global__ void __launch_bounds__(256) k_ghost_combine(int n, const long *__rest
   out[q] = mul ? mul[q] * v : v;
 }
 
-// x[fluid] += alpha (alpha read from device memory: scale * src[0] (+ scale2*src[1]))
+// x[fluid] += alpha
 __global__ void __launch_bounds__(256) k_fluid_shift(RefArgs R, LevelArgs<double> L, double *__restrict__ x,
-                                                     const double *__restrict__ num, const double *__restrict__ den,
-                                                     double sign) {
+                                                     double alpha) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   int j = blockIdx.y * blockDim.y + threadIdx.y, k = blockIdx.z;
   if (i >= R.nxc || j >= R.nyc) return;
   long a = lidx(L.sx, L.sxy, i, j, k);
   if (L.fl[a] & FL_BLANK) return;
   long r = ridx(R, i, j, k);
-  x[r] = x[r] + sign * (num[0] / den[0]);
+  x[r] = x[r] + alpha;
 }
 
 // subtracting_average_pressure body (CORE_POISSON.F90:447-457):
@@ -1962,7 +1990,8 @@ __global__ void __launch_bounds__(64 * kCoarseMaxWaves) k_coarse_mv(int n, const
 constexpr int KRY_MAX = 16;
 struct KryVecs {
   const double *u[KRY_MAX + 1];
-  double c[KRY_MAX + 1];
+  double c[KRY_MAX + 1];  // coefficients of an update
+  const double *cd;       // coefficients of an orthogonalisation (device)
   int n;
 };
 
@@ -1985,6 +2014,47 @@ __device__ inline void block_sums_to(double (&v)[KRY_MAX + 1], int n, double *s,
     double r = 0.0;
     for (int ww = 0; ww < NT / 64; ww++) r += s[ww * (KRY_MAX + 1) + tid];
     part[blk * n + tid] = r;
+  }
+}
+
+// nq <= KRY_MAX + 1 independent sums of per-workgroup partials part[b*nq +
+// q], see k_reduce_summax; 256 threads.  coef (may be null) takes s2.c[q]
+// times sum q: the Gram-Schmidt coefficients of the basis, which the
+// orthogonalisation reads without a round trip to the host.
+struct RedScale {
+  double c[KRY_MAX + 1];
+};
+__global__ void __launch_bounds__(256) k_reduce_sums(const double *__restrict__ part, int nblk, int nq, int chunk,
+                                                     double *part2, unsigned *counter, double *__restrict__ out,
+                                                     double *__restrict__ hout, RedScale s2,
+                                                     double *__restrict__ coef) {
+  __shared__ double s[4 * (KRY_MAX + 1)];
+  __shared__ double fin[KRY_MAX + 1];
+  double acc[KRY_MAX + 1];
+  auto clear = [&] {
+#pragma unroll
+    for (int q = 0; q < KRY_MAX + 1; q++) acc[q] = 0.0;
+  };
+  auto add = [&](const double *p) {
+#pragma unroll
+    for (int q = 0; q < KRY_MAX + 1; q++)
+      if (q < nq) acc[q] += p[q];
+  };
+  clear();
+  const int b0 = blockIdx.x * chunk, b1 = min(nblk, b0 + chunk);
+  for (int b = b0 + threadIdx.x; b < b1; b += 256) add(part + (long)b * nq);
+  if (gridDim.x > 1) {
+    block_sums_to<256>(acc, nq, s, part2, blockIdx.x);
+    if (!last_block(counter)) return;
+    clear();
+    if (threadIdx.x < gridDim.x) add(part2 + threadIdx.x * nq);
+    if (threadIdx.x == 0) *counter = 0;
+  }
+  block_sums_to<256>(acc, nq, s, fin, 0);
+  const int q = threadIdx.x;
+  if (q < nq) {  // written by this thread in block_sums_to
+    out[q] = hout[q] = fin[q];
+    if (coef) coef[q] = s2.c[q] * fin[q];
   }
 }
 
@@ -2049,7 +2119,7 @@ __global__ void __launch_bounds__(NT) k_kry_orth(RefArgs R, LevelArgs<double> L,
       u = w[r];
 #pragma unroll
       for (int q = 0; q < KRY_MAX + 1; q++)
-        if (q < V.n) u -= V.c[q] * V.u[q][r];
+        if (q < V.n) u -= V.cd[q] * V.u[q][r];
       w[r] = u;
     }
     rhs0[a] = (TE)u;
@@ -2086,6 +2156,7 @@ __global__ void __launch_bounds__(256) k_kry_update(RefArgs R, LevelArgs<double>
 struct KryVecsF {
   const float *u[KRY_MAX + 1];
   double c[KRY_MAX + 1];
+  const double *cd;
   int n;
 };
 
@@ -2143,7 +2214,7 @@ __global__ void __launch_bounds__(NT) k_kryl_orth(LevelArgs<double> L, float *__
       double u = (double)w[a];
 #pragma unroll
       for (int q = 0; q < KRY_MAX + 1; q++)
-        if (q < V.n) u -= V.c[q] * (double)V.u[q][a];
+        if (q < V.n) u -= V.cd[q] * (double)V.u[q][a];
       uf = (float)u;
       w[a] = uf;
     }
@@ -2296,8 +2367,9 @@ __global__ void __launch_bounds__(NT) k_kryl_orth4(LevelArgs<double> L, float *_
       if (q < V.n) {
         float uq[4];
         load_chunk<float, 4>(V.u[q] + a, 4, uq);
+        const double c = V.cd[q];
 #pragma unroll
-        for (int t = 0; t < 4; t++) u[t] -= V.c[q] * (double)uq[t];
+        for (int t = 0; t < 4; t++) u[t] -= c * (double)uq[t];
       }
     }
 #pragma unroll
