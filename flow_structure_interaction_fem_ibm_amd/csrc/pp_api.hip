@@ -12,6 +12,7 @@
 
 #include "pp_kernels.h"
 #include "pp_momentum.h"
+#include "pp_pair.h"
 #include "pp_setup.h"
 
 using namespace pp;
@@ -238,6 +239,8 @@ T *split_e(pp_ctx *c) { return std::is_same<T, float>::value ? reinterpret_cast<
 template <typename T>
 T *split_rhs(pp_ctx *c) { return std::is_same<T, float>::value ? reinterpret_cast<T *>(c->sp.rhs) : nullptr; }
 template <typename T>
+T *split_res(pp_ctx *c) { return std::is_same<T, float>::value ? reinterpret_cast<T *>(c->sp.res) : nullptr; }
+template <typename T>
 T *split_nshape(pp_ctx *c) { return std::is_same<T, float>::value ? reinterpret_cast<T *>(c->sp.nshape) : nullptr; }
 
 template <typename T>
@@ -325,8 +328,8 @@ void launch_yzline(pp_ctx *c, Level &L, int lvl, int color, T omega) {
   kend(c);
 }
 
-// solved homogeneous ghost rows on a level-0 correction (one gather)
-// (spl: on the colour-split copy, whatever e)
+// solved homogeneous ghost rows on a level-0 correction e (one gather; spl:
+// e in colour-split rows)
 template <typename T>
 void ghost_sweep_level0(pp_ctx *c, T *e, bool spl) {
   GhostTables &g = c->gh;
@@ -335,7 +338,7 @@ void ghost_sweep_level0(pp_ctx *c, T *e, bool spl) {
   double nnz = (double)g.h_c_ref.size();
   kbegin(c, PP_K_GHOST, 0, g.n * (12.0 + sizeof(T)) + nnz * (8.0 + 2.0 * sizeof(T)));
   k_ghost_composite<T, T><<<grid, block, 0, c->stream>>>(g.n, spl ? g.g_as : g.g_al, g.c_ptr, spl ? g.c_as : g.c_al,
-                                                          ghost_cw<T>(g), nullptr, spl ? split_e<T>(c) : e);
+                                                          ghost_cw<T>(g), nullptr, e);
   kend(c);
 }
 
@@ -379,10 +382,6 @@ void adj_ghost_level0(pp_ctx *c, T *e, T *rhs) {
   // on the colour-split copy while it is in use
   const bool spl = split_on<T>(c, 0);
   const long *nb = spl ? g.nb_as : g.nb_al, *ct = spl ? g.ct_as : g.ct_al;
-  if (spl) {
-    e = split_e<T>(c);
-    rhs = split_rhs<T>(c);
-  }
   dim3 grid((g.n + 255) / 256), block(256);
   const double nnz = (double)g.h_ct_ghost.size();
   kbegin(c, PP_K_GHOST, 0, g.n * 6.0 * (8 + sizeof(T)) + g.n * sizeof(T) +
@@ -414,13 +413,85 @@ void ghost_step_level0(pp_ctx *c, T *e, T *rhs) {
   else ghost_sweep_level0<T>(c, e, split_on<T>(c, 0));
 }
 
-// one zebra line pass set: x, y, z lines, two colours each
+// Levels whose two colours run in one launch per direction (pp_pair.h).
+template <typename T>
+bool pair_level(const pp_ctx *c, const Level &L, bool spl) {
+  return pair_cells(L) && (!spl || c->sp.res);
+}
+
+// both colours of the lines along dir, src -> dst
+template <typename T>
+void launch_pair(pp_ctx *c, int l, int dir, const T *src, T *dst, T omega) {
+  Level &L = c->lv[l];
+  const bool spl = split_on<T>(c, l);
+  const LevelArgs<T> a = spl ? split_args<T>(c, L) : largs<T>(L);
+  const T *rhs = spl ? split_rhs<T>(c) : lv_rhs<T>(L);
+  const int hp = c->sp.hp;
+  hipStream_t st = c->stream;
+  kbegin(c, PP_K_XLINE + dir, l, (double)L.cx * L.cy * L.cz * bytes_line(sizeof(T)));
+  auto layouts = [&](auto fn) {
+    if constexpr (std::is_same<T, float>::value) {
+      if (spl) {
+        fn(std::true_type{});
+        return;
+      }
+    }
+    fn(std::false_type{});
+  };
+  using std::integral_constant;
+  const int n = dir == 0 ? L.cx : (dir == 1 ? L.cy : L.cz), na = dir == 0 ? L.cy : L.cx, nb = dir == 2 ? L.cy : L.cz;
+  const dim3 grid((na + kPairA - 1) / kPairA, (nb + kPairB - 1) / kPairB);
+  auto go = [&](auto ls) {
+    constexpr int LS = decltype(ls)::value;
+    layouts([&](auto sp) {
+      constexpr bool SPL = decltype(sp)::value;
+      if (dir == 0) k_line_pair<T, LS, 0, SPL><<<grid, kPairThreads, 0, st>>>(a, hp, rhs, src, dst, omega);
+      else if (dir == 1) k_line_pair<T, LS, 1, SPL><<<grid, kPairThreads, 0, st>>>(a, hp, rhs, src, dst, omega);
+      else k_line_pair<T, LS, 2, SPL><<<grid, kPairThreads, 0, st>>>(a, hp, rhs, src, dst, omega);
+    });
+  };
+  if (n <= 16) go(integral_constant<int, 1>{});
+  else if (n <= 32) go(integral_constant<int, 2>{});
+  else go(integral_constant<int, 4>{});
+  kend(c);
+}
+
+// one line smoothing step: x, y, z lines, two colours each.  On pair levels
+// the correction goes back and forth between buf[0] (the level's e) and
+// buf[1], cur says where it is; with last it ends in buf[0]: an odd number
+// of launches pending then takes the z lines in place.
+template <typename T>
+void line_step(pp_ctx *c, int l, T omega, T *const buf[2], int &cur, bool last) {
+  Level &L = c->lv[l];
+  if (!pair_level<T>(c, L, split_on<T>(c, l))) {
+    for (int col = 0; col < 2; col++) launch_xline<T>(c, L, l, col, omega);
+    for (int col = 0; col < 2; col++) launch_yzline<T, 1>(c, L, l, col, omega);
+    for (int col = 0; col < 2; col++) launch_yzline<T, 2>(c, L, l, col, omega);
+    return;
+  }
+  const bool in_place = last && cur == 0;
+  for (int dir = 0; dir < (in_place ? 2 : 3); dir++, cur ^= 1) launch_pair<T>(c, l, dir, buf[cur], buf[1 - cur], omega);
+  if (in_place)
+    for (int col = 0; col < 2; col++) launch_yzline<T, 2>(c, L, l, col, omega);
+}
+
+// a level's correction and the array that its smoothing may use beside it
+template <typename T>
+struct SmoothBuf {
+  T *b[2];
+  SmoothBuf(pp_ctx *c, int l) {
+    const bool spl = split_on<T>(c, l);
+    b[0] = spl ? split_e<T>(c) : lv_e<T>(c->lv[l]);
+    b[1] = spl ? split_res<T>(c) : lv_res<T>(c->lv[l]);
+  }
+};
+
+// one step without ghost rows
 template <typename T>
 void line_passes(pp_ctx *c, int l, T omega) {
-  Level &L = c->lv[l];
-  for (int col = 0; col < 2; col++) launch_xline<T>(c, L, l, col, omega);
-  for (int col = 0; col < 2; col++) launch_yzline<T, 1>(c, L, l, col, omega);
-  for (int col = 0; col < 2; col++) launch_yzline<T, 2>(c, L, l, col, omega);
+  const SmoothBuf<T> buf(c, l);
+  int cur = 0;
+  line_step<T>(c, l, omega, buf.b, cur, true);
 }
 
 // one point-Jacobi sweep src -> dst on level l
@@ -445,24 +516,27 @@ void jacobi_pass(pp_ctx *c, int l, const T *src, T *dst, T omega) {
 // Point Jacobi alternates between e and the level's residual buffer (free
 // while smoothing) and copies back after an odd count.
 template <typename T>
-void smooth_steps(pp_ctx *c, int l, const pp_solve_opts *o, int steps, bool ghosts = true, bool zero_first = false) {
+void smooth_steps(pp_ctx *c, int l, const pp_solve_opts *o, int steps, int &cur, bool last, bool ghosts = true,
+                  bool zero_first = false) {
   Level &L = c->lv[l];
   const T om = (T)o->omega;
   if (o->smoother != PP_SMOOTH_POINT_JACOBI) {
+    const SmoothBuf<T> buf(c, l);
+    T *rhs = split_on<T>(c, l) ? split_rhs<T>(c) : lv_rhs<T>(L);
     for (int s = 0; s < steps; s++) {
-      if (l == 0 && ghosts && !(s == 0 && zero_first)) ghost_step_level0<T>(c, lv_e<T>(L), lv_rhs<T>(L));
-      line_passes<T>(c, l, om);
+      if (l == 0 && ghosts && !(s == 0 && zero_first)) ghost_step_level0<T>(c, buf.b[cur], rhs);
+      line_step<T>(c, l, om, buf.b, cur, last && s + 1 == steps);
     }
     return;
   }
   T *buf[2] = {lv_e<T>(L), lv_res<T>(L)};
-  int cur = 0;
+  int jc = 0;
   for (int s = 0; s < steps; s++) {
-    if (l == 0 && ghosts && !(s == 0 && zero_first)) ghost_step_level0<T>(c, buf[cur], lv_rhs<T>(L));
-    jacobi_pass<T>(c, l, buf[cur], buf[1 - cur], om);
-    cur ^= 1;
+    if (l == 0 && ghosts && !(s == 0 && zero_first)) ghost_step_level0<T>(c, buf[jc], lv_rhs<T>(L));
+    jacobi_pass<T>(c, l, buf[jc], buf[1 - jc], om);
+    jc ^= 1;
   }
-  if (cur) {
+  if (jc) {
     kbegin(c, PP_K_JACOBI, l, 2.0 * sizeof(T) * L.total);
     hipMemcpyAsync(buf[0], buf[1], sizeof(T) * L.total, hipMemcpyDeviceToDevice, c->stream);
     kend(c);
@@ -471,14 +545,14 @@ void smooth_steps(pp_ctx *c, int l, const pp_solve_opts *o, int steps, bool ghos
 
 // level residual res = rhs - L e (four cells per thread when rows allow)
 template <typename T>
-void launch_residual(pp_ctx *c, Level &L) {
+void launch_residual(pp_ctx *c, Level &L, const T *e) {
   LevelArgs<T> a = largs<T>(L);
   if (L.cx % 4 == 0) {
     CellLaunch q = cell_launch(L.cx / 4, L.cy, L.cz);
-    k_residual4<T><<<q.grid, q.block, 0, c->stream>>>(a, lv_e<T>(L), lv_rhs<T>(L), lv_res<T>(L));
+    k_residual4<T><<<q.grid, q.block, 0, c->stream>>>(a, e, lv_rhs<T>(L), lv_res<T>(L));
   } else {
     CellLaunch cl = cell_launch(L.cx, L.cy, L.cz);
-    k_residual<T><<<cl.grid, cl.block, 0, c->stream>>>(a, lv_e<T>(L), lv_rhs<T>(L), lv_res<T>(L));
+    k_residual<T><<<cl.grid, cl.block, 0, c->stream>>>(a, e, lv_rhs<T>(L), lv_res<T>(L));
   }
 }
 
@@ -487,11 +561,11 @@ bool halves_by2(const Level &L, const Level &C) {
   return C.cf[0] == 2 && C.cf[1] == 2 && C.cf[2] == 2 && L.cx == 2 * C.cx && L.cy == 2 * C.cy && L.cz == 2 * C.cz;
 }
 
-// residual of level l restricted onto level l + 1 (its rhs; its correction
-// zeroed): one fused pass where the level halves in all three directions,
+// residual of the correction e of level l restricted onto level l + 1 (its
+// rhs; its correction zeroed): one fused pass where the level halves in all three directions,
 // else the level residual and the general restriction
 template <typename T>
-void restrict_step(pp_ctx *c, int l) {
+void restrict_step(pp_ctx *c, int l, const T *e) {
   Level &L = c->lv[l], &C = c->lv[l + 1];
   hipStream_t st = c->stream;
   const double cells = (double)L.cx * L.cy * L.cz;
@@ -500,16 +574,16 @@ void restrict_step(pp_ctx *c, int l) {
   if (split_on<T>(c, l)) {
     // Split0::ok guarantees the by-2 halving
     kbegin(c, PP_K_RESTRICT, l, cells * (2.0 * sizeof(T) + 1.0) + 2.0 * sizeof(T) * C.cx * C.cy * C.cz);
-    k_resrestrict2<T, true><<<cc.grid, cc.block, 0, st>>>(split_args<T>(c, L), ac, split_e<T>(c), split_rhs<T>(c),
+    k_resrestrict2<T, true><<<cc.grid, cc.block, 0, st>>>(split_args<T>(c, L), ac, e, split_rhs<T>(c),
                                                           lv_rhs<T>(C), lv_e<T>(C), c->sp.hp);
     kend(c);
   } else if (halves_by2(L, C)) {
     kbegin(c, PP_K_RESTRICT, l, cells * (2.0 * sizeof(T) + 1.0) + 2.0 * sizeof(T) * C.cx * C.cy * C.cz);
-    k_resrestrict2<T><<<cc.grid, cc.block, 0, st>>>(a, ac, lv_e<T>(L), lv_rhs<T>(L), lv_rhs<T>(C), lv_e<T>(C), 0);
+    k_resrestrict2<T><<<cc.grid, cc.block, 0, st>>>(a, ac, e, lv_rhs<T>(L), lv_rhs<T>(C), lv_e<T>(C), 0);
     kend(c);
   } else {
     kbegin(c, PP_K_RESIDUAL, l, cells * (3.0 * sizeof(T) + 1.0));
-    launch_residual<T>(c, L);
+    launch_residual<T>(c, L, e);
     kend(c);
     kbegin(c, PP_K_RESTRICT, l, cells * (sizeof(T) + 1.0) + 2.0 * sizeof(T) * C.cx * C.cy * C.cz);
     k_restrict<T><<<cc.grid, cc.block, 0, st>>>(a, ac, C.cf[0], C.cf[1], C.cf[2], lv_res<T>(L), lv_rhs<T>(C),
@@ -526,9 +600,9 @@ template <>
 const double *nshape<double>(pp_ctx *c) { return c->d_nshape64; }
 
 // the correction of level l + 1 prolongated onto level l and added to its
-// correction on fluid cells
+// correction e on fluid cells
 template <typename T>
-void prolong_step(pp_ctx *c, int l) {
+void prolong_step(pp_ctx *c, int l, T *e) {
   Level &L = c->lv[l], &C = c->lv[l + 1];
   hipStream_t st = c->stream;
   const double cells = (double)L.cx * L.cy * L.cz;
@@ -541,16 +615,16 @@ void prolong_step(pp_ctx *c, int l) {
     CellLaunch cc = cell_launch(C.cx, C.cy, C.cz);
     const T *sscale = scale ? (const T *)split_nshape<T>(c) : nullptr;
     k_prolong2<T, true><<<cc.grid, cc.block, 0, st>>>(split_args<T>(c, L), ac, pdir<T>(L, 0).wpar,
-                                                      pdir<T>(L, 1).wpar, pdir<T>(L, 2).wpar, lv_e<T>(C),
-                                                      split_e<T>(c), sscale, c->sp.hp);
+                                                      pdir<T>(L, 1).wpar, pdir<T>(L, 2).wpar, lv_e<T>(C), e,
+                                                      sscale, c->sp.hp);
   } else if (halves_by2(L, C)) {
     CellLaunch cc = cell_launch(C.cx, C.cy, C.cz);
     k_prolong2<T><<<cc.grid, cc.block, 0, st>>>(a, ac, pdir<T>(L, 0).wpar, pdir<T>(L, 1).wpar, pdir<T>(L, 2).wpar,
-                                                 lv_e<T>(C), lv_e<T>(L), scale, 0);
+                                                 lv_e<T>(C), e, scale, 0);
   } else {
     CellLaunch cl = cell_launch(L.cx, L.cy, L.cz);
-    k_prolong<T><<<cl.grid, cl.block, 0, st>>>(a, ac, pdir<T>(L, 0), pdir<T>(L, 1), pdir<T>(L, 2), lv_e<T>(C),
-                                                lv_e<T>(L), scale);
+    k_prolong<T><<<cl.grid, cl.block, 0, st>>>(a, ac, pdir<T>(L, 0), pdir<T>(L, 1), pdir<T>(L, 2), lv_e<T>(C), e,
+                                                scale);
   }
   kend(c);
 }
@@ -580,11 +654,15 @@ void vcycle(pp_ctx *c, int l, const pp_solve_opts *o) {
   // level-0 correction (every caller zeroes it)
   const bool zero = l == 0 && c->e0_zero;
   if (l == 0) c->e0_zero = false;
-  smooth_steps<T>(c, l, o, npre, true, zero);
-  restrict_step<T>(c, l);
+  // where the correction lies (SmoothBuf); the general restriction needs the
+  // level's second array, and every cycle leaves it in the first
+  const SmoothBuf<T> buf(c, l);
+  int cur = 0;
+  smooth_steps<T>(c, l, o, npre, cur, npost == 0 || !halves_by2(L, c->lv[l + 1]), true, zero);
+  restrict_step<T>(c, l, buf.b[cur]);
   vcycle<T>(c, l + 1, o);
-  prolong_step<T>(c, l);
-  smooth_steps<T>(c, l, o, npost);
+  prolong_step<T>(c, l, buf.b[cur]);
+  smooth_steps<T>(c, l, o, npost, cur, true);
 }
 
 // FP32 line-smoothed cycles run level 0 on its colour-split copy.
@@ -1024,7 +1102,7 @@ struct FwdOps32 {
     Level &L0 = c->lv[0];
     CellLaunch cl = launch();
     const bool spl = sio();
-    ghost_sweep_level0<float>(c, lv_e<float>(L0), spl);
+    ghost_sweep_level0<float>(c, spl ? c->sp.e : lv_e<float>(L0), spl);
     kbegin(c, PP_K_KRYLOV, 0, cells * (4.0 + 1.0 + 4.0 + 4.0 + 4.0 * (j + 1)));
     if (spl)
       k_kryl_apply4<256, true><<<cl.grid, cl.block, 0, c->stream>>>(largs<double>(L0), c->sp.e, z(j), u(j + 1), vv,
@@ -2233,7 +2311,7 @@ int time_kernel(pp_ctx *c, int cls, int level, int reps, double *avg_us, double 
       case PP_K_ZLINE: launch_yzline<T, 2>(c, L, level, r & 1, T(1)); break;
       default:
         kbegin(c, PP_K_RESIDUAL, level, (double)L.cx * L.cy * L.cz * (3.0 * sizeof(T) + 1.0));
-        launch_residual<T>(c, L);
+        launch_residual<T>(c, L, lv_e<T>(L));
         kend(c);
         break;
     }
@@ -2333,7 +2411,7 @@ int level_apply(pp_ctx *c, int op, int l, double omega, const double *a, const d
   switch (op) {
     case PP_LOP_RESIDUAL:
       if ((rc = level_upload<T>(c, L, a, lv_e<T>(L))) || (rc = level_upload<T>(c, L, b, lv_rhs<T>(L)))) return rc;
-      launch_residual<T>(c, L);
+      launch_residual<T>(c, L, lv_e<T>(L));
       return level_download<T>(c, L, lv_res<T>(L), out);
     case PP_LOP_RESTRICT: {
       Level &C = c->lv[l + 1];
@@ -2345,13 +2423,13 @@ int level_apply(pp_ctx *c, int op, int l, double omega, const double *a, const d
     }
     case PP_LOP_RESRESTRICT:
       if ((rc = level_upload<T>(c, L, a, lv_e<T>(L))) || (rc = level_upload<T>(c, L, b, lv_rhs<T>(L)))) return rc;
-      restrict_step<T>(c, l);
+      restrict_step<T>(c, l, lv_e<T>(L));
       return level_download<T>(c, c->lv[l + 1], lv_rhs<T>(c->lv[l + 1]), out);
     case PP_LOP_PROLONG:
       if ((rc = level_upload<T>(c, c->lv[l + 1], a, lv_e<T>(c->lv[l + 1]))) ||
           (rc = level_upload<T>(c, L, b, lv_e<T>(L))))
         return rc;
-      prolong_step<T>(c, l);
+      prolong_step<T>(c, l, lv_e<T>(L));
       return level_download<T>(c, L, lv_e<T>(L), out);
     default:  // PP_LOP_LINE_PASS
       if ((rc = level_upload<T>(c, L, a, lv_e<T>(L))) || (rc = level_upload<T>(c, L, b, lv_rhs<T>(L)))) return rc;
@@ -2426,7 +2504,8 @@ int32_t pp_smooth(pp_ctx *c, int32_t smoother, double omega, int32_t sweeps, dou
   o.omega = omega;
   const bool adj = c->adjoint_mode;
   c->adjoint_mode = false;
-  smooth_steps<double>(c, 0, &o, sweeps, false);
+  int cur = 0;
+  smooth_steps<double>(c, 0, &o, sweeps, cur, true, false);
   c->adjoint_mode = adj;
   k_level_to_ref<double><<<cl.grid, cl.block, 0, c->stream>>>(c->ref, a, L.e64, c->d_p);
   HIPCHK(hipGetLastError());

@@ -125,7 +125,7 @@ void free_levels(pp_ctx *c) {
     hipFree(L.e64); hipFree(L.rhs64); hipFree(L.res64);
   }
   c->lv.clear();
-  hipFree(c->sp.e); hipFree(c->sp.rhs); hipFree(c->sp.fl); hipFree(c->sp.nshape);
+  hipFree(c->sp.e); hipFree(c->sp.rhs); hipFree(c->sp.fl); hipFree(c->sp.nshape); hipFree(c->sp.res);
   c->sp = Split0();
 }
 
@@ -341,7 +341,7 @@ __global__ void k_flags_split(int cx, int cy, int cz, int sx, long sxy, const ui
 // 128-byte line).
 int setup_split0(pp_ctx *c) {
   Split0 &sp = c->sp;
-  hipFree(sp.e); hipFree(sp.rhs); hipFree(sp.fl); hipFree(sp.nshape);
+  hipFree(sp.e); hipFree(sp.rhs); hipFree(sp.fl); hipFree(sp.nshape); hipFree(sp.res);
   sp = Split0();
   if (c->lv.size() < 2) return PP_OK;
   const Level &L = c->lv[0], &C = c->lv[1];
@@ -366,6 +366,10 @@ int setup_split0(pp_ctx *c) {
   sp.total = sp.sxy * (L.cz + 2);
   if (hipMalloc(&sp.e, sp.total * 4) != hipSuccess || hipMalloc(&sp.rhs, sp.total * 4) != hipSuccess ||
       hipMalloc(&sp.nshape, sp.total * 4) != hipSuccess || hipMalloc(&sp.fl, sp.total) != hipSuccess) {
+    set_error("hipMalloc failed for the colour-split level 0 (%ld cells)", sp.total);
+    return PP_HIP_ERROR;
+  }
+  if (pair_cells(L) && (hipMalloc(&sp.res, sp.total * 4) != hipSuccess || hipMemset(sp.res, 0, sp.total * 4) != hipSuccess)) {
     set_error("hipMalloc failed for the colour-split level 0 (%ld cells)", sp.total);
     return PP_HIP_ERROR;
   }
