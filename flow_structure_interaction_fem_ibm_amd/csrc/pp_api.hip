@@ -244,7 +244,7 @@ template <typename T>
 T *split_nshape(pp_ctx *c) { return std::is_same<T, float>::value ? reinterpret_cast<T *>(c->sp.nshape) : nullptr; }
 
 template <typename T>
-void launch_xline(pp_ctx *c, Level &L, int lvl, int color, T omega) {
+void launch_xline(pp_ctx *c, Level &L, int lvl, int color, T omega, bool zero = false) {
   const bool spl = split_on<T>(c, lvl);
   LevelArgs<T> a = spl ? split_args<T>(c, L) : largs<T>(L);
   int G, S;
@@ -261,11 +261,11 @@ void launch_xline(pp_ctx *c, Level &L, int lvl, int color, T omega) {
     // the split layout needs even chunks (Split0::ok guarantees them)
     if constexpr (SS % 2 == 0 && std::is_same<T, float>::value) {
       if (spl) {
-        k_xline<T, GG, SS, true><<<grid, block, 0, st>>>(a, rhs, e, color, omega, hp);
+        k_xline<T, GG, SS, true><<<grid, block, 0, st>>>(a, rhs, e, color, omega, hp, zero);
         return;
       }
     }
-    k_xline<T, GG, SS><<<grid, block, 0, st>>>(a, rhs, e, color, omega, 0);
+    k_xline<T, GG, SS><<<grid, block, 0, st>>>(a, rhs, e, color, omega, 0, zero);
   });
   kend(c);
 }
@@ -459,12 +459,13 @@ void launch_pair(pp_ctx *c, int l, int dir, const T *src, T *dst, T omega) {
 // one line smoothing step: x, y, z lines, two colours each.  On pair levels
 // the correction goes back and forth between buf[0] (the level's e) and
 // buf[1], cur says where it is; with last it ends in buf[0]: an odd number
-// of launches pending then takes the z lines in place.
+// of launches pending then takes the z lines in place.  zero: the correction
+// is zero on entry (launch_xline; pair levels need it zero in memory).
 template <typename T>
-void line_step(pp_ctx *c, int l, T omega, T *const buf[2], int &cur, bool last) {
+void line_step(pp_ctx *c, int l, T omega, T *const buf[2], int &cur, bool last, bool zero = false) {
   Level &L = c->lv[l];
   if (!pair_level<T>(c, L, split_on<T>(c, l))) {
-    for (int col = 0; col < 2; col++) launch_xline<T>(c, L, l, col, omega);
+    for (int col = 0; col < 2; col++) launch_xline<T>(c, L, l, col, omega, zero);
     for (int col = 0; col < 2; col++) launch_yzline<T, 1>(c, L, l, col, omega);
     for (int col = 0; col < 2; col++) launch_yzline<T, 2>(c, L, l, col, omega);
     return;
@@ -525,7 +526,7 @@ void smooth_steps(pp_ctx *c, int l, const pp_solve_opts *o, int steps, int &cur,
     T *rhs = split_on<T>(c, l) ? split_rhs<T>(c) : lv_rhs<T>(L);
     for (int s = 0; s < steps; s++) {
       if (l == 0 && ghosts && !(s == 0 && zero_first)) ghost_step_level0<T>(c, buf.b[cur], rhs);
-      line_step<T>(c, l, om, buf.b, cur, last && s + 1 == steps);
+      line_step<T>(c, l, om, buf.b, cur, last && s + 1 == steps, zero_first && s == 0);
     }
     return;
   }
@@ -650,9 +651,9 @@ void vcycle(pp_ctx *c, int l, const pp_solve_opts *o) {
   }
   const int npre = (l > 0 && o->nu_coarse > 0) ? o->nu_coarse : o->nu_pre;
   const int npost = (l > 0 && o->nu_coarse > 0) ? o->nu_coarse : o->nu_post;
-  // the first cycle of a preconditioner application starts from a zero
-  // level-0 correction (every caller zeroes it)
-  const bool zero = l == 0 && c->e0_zero;
+  // the first cycle of a preconditioner application starts from a zero level-0
+  // correction, the coarser levels always do (restrict_step zeroes theirs)
+  const bool zero = l > 0 || c->e0_zero;
   if (l == 0) c->e0_zero = false;
   // where the correction lies (SmoothBuf); the general restriction needs the
   // level's second array, and every cycle leaves it in the first
@@ -670,12 +671,16 @@ template <typename T>
 bool split_cycles(const pp_ctx *c, const pp_solve_opts *o) {
   return std::is_same<T, float>::value && c->sp.ok && o->smoother == PP_SMOOTH_LINE;
 }
-void split_in(pp_ctx *c) {
+// Their first pass takes the correction as zero without reading it.
+bool split_zero_unread(const pp_ctx *c, const pp_solve_opts *o) {
+  return o->nu_pre > 0 && !pair_level<float>(c, c->lv[0], true);
+}
+void split_in(pp_ctx *c, const pp_solve_opts *o) {
   Level &L0 = c->lv[0];
   const CellLaunch q = cell_launch((L0.cx + 1) / 2, L0.cy, L0.cz);
   kbegin(c, PP_K_OTHER, 0, (double)L0.cx * L0.cy * L0.cz * 12.0);
   k_split_in<<<q.grid, q.block, 0, c->stream>>>(largs<float>(L0), split_args<float>(c, L0), c->sp.hp, L0.rhs32,
-                                                c->sp.rhs, c->sp.e);
+                                                c->sp.rhs, split_zero_unread(c, o) ? nullptr : c->sp.e);
   kend(c);
 }
 void split_out(pp_ctx *c) {
@@ -698,7 +703,7 @@ template <typename T>
 void precondition_cycles(pp_ctx *c, const pp_solve_opts *o, bool in_split = false, bool out_split = false) {
   const bool spl = split_cycles<T>(c, o);
   if (spl) {
-    if (!in_split) split_in(c);
+    if (!in_split) split_in(c, o);
     c->sp.on = true;
   }
   c->e0_zero = true;
@@ -717,7 +722,7 @@ template <typename T>
 void adjoint_cycles(pp_ctx *c, const pp_solve_opts *o, pp_solve_stats &S, bool in_split = false,
                     bool out_split = false) {
   const bool spl = split_cycles<T>(c, o);
-  if (spl && !in_split) split_in(c);
+  if (spl && !in_split) split_in(c, o);
   adj_ghost_base<T>(c, spl);
   c->adjoint_mode = true;
   c->sp.on = spl;
@@ -1081,7 +1086,7 @@ struct FwdOps32 {
   double *p;
   bool have_bnd;
   double cells;
-  bool rhs_split = false;  // the last orth wrote the split rhs (and zeroed the split correction)
+  bool rhs_split = false;  // the last orth wrote the split rhs (and zeroed the split correction if it is read)
   float *u(int q) { return c->d_kryl[q]; }
   float *z(int q) { return c->d_kryl[c->kryl_m + 1 + q]; }
   // four cells per thread where the level-0 rows allow it
@@ -1122,8 +1127,8 @@ struct FwdOps32 {
     rhs_split = sio();
     if (rhs_split)
       k_kryl_orth4<256, true><<<cl.grid, cl.block, 0, c->stream>>>(largs<double>(L0), u(j + 1), vv, c->sp.rhs,
-                                                                   c->sp.e, c->d_part, c->sp.sx, c->sp.sxy,
-                                                                   c->sp.hp);
+                                                                   split_zero_unread(c, o) ? nullptr : c->sp.e,
+                                                                   c->d_part, c->sp.sx, c->sp.sxy, c->sp.hp);
     else if (by4())
       k_kryl_orth4<256><<<cl.grid, cl.block, 0, c->stream>>>(largs<double>(L0), u(j + 1), vv, lv_rhs<float>(L0),
                                                              lv_e<float>(L0), c->d_part, 0, 0, 0);
@@ -1440,8 +1445,8 @@ struct AdjOps32 {
     rhs_split = sio();
     if (rhs_split)
       k_kryl_orth4<256, true><<<cl.grid, cl.block, 0, c->stream>>>(largs<double>(L0), u(j + 1), vv, c->sp.rhs,
-                                                                   c->sp.e, c->d_part, c->sp.sx, c->sp.sxy,
-                                                                   c->sp.hp);
+                                                                   split_zero_unread(c, o) ? nullptr : c->sp.e,
+                                                                   c->d_part, c->sp.sx, c->sp.sxy, c->sp.hp);
     else
       k_kryl_orth4<256><<<cl.grid, cl.block, 0, c->stream>>>(largs<double>(L0), u(j + 1), vv, lv_rhs<float>(L0),
                                                              lv_e<float>(L0), c->d_part, 0, 0, 0);

@@ -1617,6 +1617,12 @@ __device__ inline int xcd_block(int b, int nb) {
 // x-line zebra pass (lines along the contiguous index): lines (j,k) with
 // (j+k)%2 == color; a group of G lanes holds one line, S cells per lane.
 // ---------------------------------------------------------------------
+// zero: the first passes on a correction that is zero whatever memory holds:
+// colour 0 reads the right-hand side alone, colour 1 no values of its own,
+// and both together write every cell of the level.  With the zeroing of the
+// split level 0 left out that takes 1.9 GB of traffic out of a 512x512x384
+// cycle: its mixed solve 79.6 -> 77.5 ms.
+//
 // SPL: the level is the finest in the colour-split row layout (sidx,
 // half-row offset hp; S even): a lane's S cells are S/2 consecutive even
 // cells and the S/2 odd cells beside them, read whole (the rows' padding and
@@ -1627,7 +1633,7 @@ __device__ inline int xcd_block(int b, int nb) {
 // cell and flag, 467 against 917 VALU instructions per wavefront.
 template <typename T, int G, int S, bool SPL = false>
 __global__ void __launch_bounds__(256) k_xline(LevelArgs<T> L, const T *__restrict__ rhs, T *__restrict__ e,
-                                               int color, T omega, int hp) {
+                                               int color, T omega, int hp, bool zero) {
   static_assert(!SPL || S % 2 == 0, "split rows need an even chunk");
   const int blk = xcd_block(blockIdx.x, gridDim.x);
   const int line = (blk * 256 + (int)threadIdx.x) / G;
@@ -1654,13 +1660,20 @@ __global__ void __launch_bounds__(256) k_xline(LevelArgs<T> L, const T *__restri
     }
   };
   const T my = L.cmy[j], py = L.cpy[j], mz = L.cmz[k], pz = L.cpz[k];
-  ld(e + base, eo);
+  const bool nbr = !zero || color != 0;
+  if (zero) {
+#pragma unroll
+    for (int s = 0; s < S; s++) eo[s] = T(0);
+  } else {
+    ld(e + base, eo);
+  }
   ld(rhs + base, rv);
   SegElim<T, S> se;
   if constexpr (SPL) {
     const long st[4] = {-(long)L.sx, L.sx, -L.sxy, L.sxy};
     const T ct[4] = {my, py, mz, pz};
-    if constexpr (S < 16) {
+    if (!nbr) {
+    } else if constexpr (S < 16) {
 #pragma unroll
       for (int t = 0; t < 4; t++) {
         T v[S];
@@ -1699,10 +1712,15 @@ __global__ void __launch_bounds__(256) k_xline(LevelArgs<T> L, const T *__restri
     }
   } else {
     T ejm[S], ejp[S], ekm[S], ekp[S];
-    ld(e + base - L.sx, ejm);
-    ld(e + base + L.sx, ejp);
-    ld(e + base - L.sxy, ekm);
-    ld(e + base + L.sxy, ekp);
+    if (nbr) {
+      ld(e + base - L.sx, ejm);
+      ld(e + base + L.sx, ejp);
+      ld(e + base - L.sxy, ekm);
+      ld(e + base + L.sxy, ekp);
+    } else {
+#pragma unroll
+      for (int s = 0; s < S; s++) ejm[s] = ejp[s] = ekm[s] = ekp[s] = T(0);
+    }
     load_chunk<T, S>(L.cmx + i0, nv, cmx);
     load_chunk<T, S>(L.cpx + i0, nv, cpx);
     load_flags<S>(L.fl + base, nv, fl);
@@ -1907,8 +1925,8 @@ __global__ void __launch_bounds__(sizeof(T) == 4 ? 1024 : 512)
   }
 }
 
-// The FP32 level-0 right-hand side into the colour-split copy, and the
-// split correction zeroed (interior cells; two cells per thread).
+// The FP32 level-0 right-hand side into the colour-split copy, and the split
+// correction zeroed unless e_s is null (interior cells; two cells per thread).
 __global__ void __launch_bounds__(256) k_split_in(LevelArgs<float> N, LevelArgs<float> S, int hp,
                                                   const float *__restrict__ rhs, float *__restrict__ rhs_s,
                                                   float *__restrict__ e_s) {
@@ -1918,10 +1936,10 @@ __global__ void __launch_bounds__(256) k_split_in(LevelArgs<float> N, LevelArgs<
   if (i >= N.cx || j >= N.cy) return;
   const long a = lidx(N.sx, N.sxy, i, j, k), se = sidx(S.sx, S.sxy, hp, i, j, k);
   rhs_s[se] = rhs[a];
-  e_s[se] = 0.f;
+  if (e_s) e_s[se] = 0.f;
   if (i + 1 < N.cx) {
     rhs_s[se + hp] = rhs[a + 1];
-    e_s[se + hp] = 0.f;
+    if (e_s) e_s[se + hp] = 0.f;
   }
 }
 
@@ -2344,7 +2362,7 @@ __global__ void __launch_bounds__(NT) k_kryl_adj_coupling(int nct, const long *_
 
 // k_kryl_orth for four consecutive cells per thread (cx % 4 == 0)
 // SPL: rhs0 and e0 are the colour-split copies (rows sp_sx, planes sp_sxy,
-// half-row offset hp); w stays in the natural layout.
+// half-row offset hp; e0 null: left as it is); w stays in the natural layout.
 template <int NT, bool SPL = false>
 __global__ void __launch_bounds__(NT) k_kryl_orth4(LevelArgs<double> L, float *__restrict__ w, KryVecsF V,
                                                    float *__restrict__ rhs0, float *__restrict__ e0,
@@ -2382,8 +2400,10 @@ __global__ void __launch_bounds__(NT) k_kryl_orth4(LevelArgs<double> L, float *_
       const long se = sidx(sp_sx, sp_sxy, hp, i0, j, k);
       *reinterpret_cast<float2 *>(rhs0 + se) = make_float2(uf[0], uf[2]);
       *reinterpret_cast<float2 *>(rhs0 + se + hp) = make_float2(uf[1], uf[3]);
-      *reinterpret_cast<float2 *>(e0 + se) = make_float2(0.0f, 0.0f);
-      *reinterpret_cast<float2 *>(e0 + se + hp) = make_float2(0.0f, 0.0f);
+      if (e0) {
+        *reinterpret_cast<float2 *>(e0 + se) = make_float2(0.0f, 0.0f);
+        *reinterpret_cast<float2 *>(e0 + se + hp) = make_float2(0.0f, 0.0f);
+      }
     } else {
       store_chunk<float, 4>(rhs0 + a, 4, uf);
       const float zero[4] = {0.0f, 0.0f, 0.0f, 0.0f};
