@@ -29,7 +29,7 @@ using namespace pp;
 // ---------------------------------------------------------------------
 // Scratch memory of the allocation-free entry point (pp_divergence_noalloc):
 // one array per GPU for the whole process, holding the per-workgroup
-// partial sums of the reduction and its two later stages.  Host code never
+// partial sums, their chunks' sums, the result and its counter.  Host code never
 // uses the array's name as an address: pp_create looks up its device
 // address once per device (hipGetSymbolAddress with the device current) and
 // the entry point passes that address to the kernels.
