@@ -2045,7 +2045,7 @@ AdSplit ad_split(const pp_ctx *c) {
   A.hp = ((c->nxc / 2 + 2 + 15) / 16) * 16;
   A.sx = SPLIT_E0 + 2 * A.hp;
   A.sxy = (long)A.sx * (c->nyc + 2);
-  A.total = A.sxy * (c->nzc + 2 + kAdMaxLS);
+  A.total = A.sxy * (c->nzc + 2);
   double *b = c->adw.buf;
   for (int q = 0; q < 3; q++) { A.var[q] = b + q * A.total; A.rw[q] = b + (3 + q) * A.total; }
   A.row = b + 6 * A.total;
@@ -2758,7 +2758,9 @@ int ad_work(pp_ctx *c, AdSplit *out) {
 // 1604).  Fewer blocks are latency-bound and want short segments: 4 cells
 // below 1024 blocks (130x98x82: 19.1-20.5 us against 19.9-20.5; 96 cells
 // cubed fill half the CUs with 16), 2 cells in 4-line tiles below 256
-// (48x40x32: 4.5-5.0 us against 6.3 with 4 cells in 16-line tiles).
+// (48x40x32: 4.5-5.0 us against 6.3 with 4 cells in 16-line tiles).  Lines
+// that fill their last segment take the passes without the test for a cell
+// past the end (256x192x192 solve: 10.96 ms, with it 11.11).
 void ad_yz_shape(int n, int half, int planes, int &LS, int &TX) {
   const long blocks = (long)((half + 15) / 16) * planes;
   if (blocks <= 256 && n <= 256) {
@@ -2779,10 +2781,16 @@ void ad_launch_yz(pp_ctx *c, const AdSplit &A, int color) {
   const dim3 grid((half + TX - 1) / TX, planes), block(TX, P);
   const size_t lds = sizeof(double2) * 6 * (size_t)(TX * P + 1);
   hipStream_t s = c->stream;
+  auto go = [&](auto ls) {
+    constexpr int L = decltype(ls)::value;
+    if (n % L) k_ad_yzline<DIR, L, true><<<grid, block, lds, s>>>(A, color);
+    else k_ad_yzline<DIR, L, false><<<grid, block, lds, s>>>(A, color);
+  };
+  using std::integral_constant;
   switch (LS) {
-    case 2: k_ad_yzline<DIR, 2><<<grid, block, lds, s>>>(A, color); break;
-    case 4: k_ad_yzline<DIR, 4><<<grid, block, lds, s>>>(A, color); break;
-    default: k_ad_yzline<DIR, kAdMaxLS><<<grid, block, lds, s>>>(A, color); break;
+    case 2: go(integral_constant<int, 2>{}); break;
+    case 4: go(integral_constant<int, 4>{}); break;
+    default: go(integral_constant<int, kAdMaxLS>{}); break;
   }
 }
 
@@ -2793,8 +2801,10 @@ void ad_launch_x(pp_ctx *c, const AdSplit &A, int color) {
   const long lines = (long)((A.cy + 1) / 2) * A.cz;
   const int nt = lines * P <= 256L * 256 ? 64 : 256;
   const int TX = std::max(1, nt / P);
-  k_ad_xline<<<(unsigned)((lines + TX - 1) / TX), TX * P, sizeof(double2) * 6 * (size_t)(TX * P + 1), c->stream>>>(
-      A, color, P, TX);
+  const unsigned grid = (unsigned)((lines + TX - 1) / TX);
+  const size_t lds = sizeof(double2) * 6 * (size_t)(TX * P + 1);
+  if (A.cx % 4) k_ad_xline<true><<<grid, TX * P, lds, c->stream>>>(A, color, P, TX);
+  else k_ad_xline<false><<<grid, TX * P, lds, c->stream>>>(A, color, P, TX);
 }
 
 // Fresh cells (fluid now, blank at the previous geometry) take the

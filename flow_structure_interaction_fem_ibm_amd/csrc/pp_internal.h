@@ -179,7 +179,7 @@ struct FreshRows {
 // rows, allocated at the first momentum call and kept with the context.
 struct AdWork {
   int hp = 0, sx = 0;
-  long sxy = 0, total = 0;     // values per array, spare identity planes included
+  long sxy = 0, total = 0;     // values per array
   double *buf = nullptr;       // 13 arrays of total values: var 3, rw 3, row 7
 };
 

@@ -12,16 +12,18 @@
 // The copy carries what the passes would otherwise test per cell: row
 // coefficients across a closed face are 0, a blank row is the identity
 // (coefficients 0, diagonal 1) with right-hand side 0, or on a ghost cell
-// its current value, so the passes read no flags.  Halo rows and the padding
-// are identity rows too.
+// its current value, so the passes read no flags.  The outer layer holds the
+// caller's values, whose edges and corners only the ghost and fresh-cell
+// stencils read: a line's rows end with its last cell, and what a segment
+// covers behind it is the literal identity row (a row of zero coefficients
+// would still take 0 * x from its neighbours, NaN where those are not finite).
 #pragma once
 
 #include "pp_kernels.h"
 
 namespace pp {
 
-// longest segment of a y/z line per thread (spare identity planes at the end
-// of the copies)
+// longest segment of a y/z line per thread
 constexpr int kAdMaxLS = 16;
 
 // Split-row geometry and arrays of the momentum solve: total values per
@@ -211,8 +213,8 @@ __device__ inline void ad_reduced_solve(double2 *sh, int nslot, int slot, int ss
 // == colour, i.e. one contiguous half of each row; a block of TX lines x P
 // segments of LS cells.  The three fields share the row coefficients and are
 // independent until the ghost update, so one pass gives what three would.
-// The copies end in LS spare identity planes, so the cells a last segment
-// reads past its line are identity rows or belong behind one.
+// Past a line's end (RAG: segments reach there) a segment reads its first
+// cell again, for rows that are then replaced by the identity.
 // ---------------------------------------------------------------------
 //
 // Bound by HBM: 64 B/cell (half of the seven row coefficients 28 and of the
@@ -222,7 +224,7 @@ __device__ inline void ad_reduced_solve(double2 *sh, int nslot, int slot, int ss
 // taken one at a time (see below), so that several blocks share a CU.
 // 256x192x192: 150 us, 4.0 TB/s, against 387 (y) and 401 us (z) in the
 // caller's layout with one block per CU and flag tests.
-template <int DIR, int LS>
+template <int DIR, int LS, bool RAG>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 8))) k_ad_yzline(AdSplit A, int color) {
   extern __shared__ unsigned char smem_raw[];
   const int TX = blockDim.x, P = blockDim.y;
@@ -247,15 +249,17 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 8))
   SegElimN<double, LS, 3> se;
 #pragma unroll
   for (int m = 0; m < LS; m++) {
-    const long o = v + m * lstr;
+    const bool in = !RAG || m0 + m < n;  // m0 < n
+    const long o = in ? v + m * lstr : v;
     const double axm = cxm[o], axp = cxp[o], aom = com[o], aop = cop[o];
     double d[3];
 #pragma unroll
     for (int q = 0; q < 3; q++) {
       const double *x = A.var[q] + base;
-      d[q] = A.rw[q][base + o] - x[o + dlo] * axm - x[o + dhi] * axp - x[o - ostr] * aom - x[o + ostr] * aop;
+      const double r = A.rw[q][base + o] - x[o + dlo] * axm - x[o + dhi] * axp - x[o - ostr] * aom - x[o + ostr] * aop;
+      d[q] = in ? r : 0.0;
     }
-    se.push(m, clm[o], cd[o], clp[o], d);
+    se.push(m, in ? clm[o] : 0.0, in ? cd[o] : 1.0, in ? clp[o] : 0.0, d);
     // the row's results are needed here, before the next cell's loads: left
     // alone the compiler loads the whole segment first (190 registers at
     // LS = 4, one block per CU, 204 us against 175 with LS = 4 this way)
@@ -280,6 +284,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 8))
 // 130 us, 4.65 TB/s on the 64 B/cell it must move, against 471 us with
 // single 8-byte loads 32 bytes apart per lane and an LDS layout whose
 // neighbouring equations met in the same banks.
+template <bool RAG>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 8)))
 k_ad_xline(AdSplit A, int color, int P, int TX) {
   extern __shared__ unsigned char smem_raw[];
@@ -320,8 +325,9 @@ k_ad_xline(AdSplit A, int color, int P, int TX) {
   SegElimN<double, 4, 3> se;
 #pragma unroll
   for (int m = 0; m < 4; m++) {
-    const double dm[3] = {d[0][m], d[1][m], d[2][m]};
-    se.push(m, a[m], b[m], c[m], dm);
+    const bool in = !RAG || 4 * seg + m < A.cx;
+    const double dm[3] = {in ? d[0][m] : 0.0, in ? d[1][m] : 0.0, in ? d[2][m] : 0.0};
+    se.push(m, in ? a[m] : 0.0, in ? b[m] : 1.0, in ? c[m] : 0.0, dm);
   }
   double XL[3], XS[3];
   ad_reduced_solve<4>(reinterpret_cast<double2 *>(smem_raw), TX * P, threadIdx.x, 1, P, seg, se, XL, XS);
