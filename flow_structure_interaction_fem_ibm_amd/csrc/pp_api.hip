@@ -2851,8 +2851,8 @@ void ad_sweeps(pp_ctx *c, const AdSplit &A, const FreshCorr *fc) {
   for (int dir = 0; dir < 3; dir++)
     for (int color = 0; color < 2; color++) {
       if (fc)
-        k_fresh_rhs<<<(3 * c->fr.n + 255) / 256, 256, 0, c->stream>>>(c->fr.n, 3, c->fr.ids, c->fr.ids_s,
-                                                                      c->fr.coff_s, c->fr.cc, *fc);
+        k_fresh_rhs<<<(3 * c->fr.n + 255) / 256, 256, 0, c->stream>>>(c->fr.n, 3, c->d_iblank_ref, c->fr.ids,
+                                                                      c->fr.ids_s, c->fr.coff_s, c->fr.cc, *fc);
       if (dir == 0) ad_launch_x(c, A, color);
       else if (dir == 1) ad_launch_yz<1>(c, A, color);
       else ad_launch_yz<2>(c, A, color);
@@ -3121,7 +3121,8 @@ int32_t solve_ad_run(pp_ctx *c, int32_t advec_scheme, double *d_u, double *d_v, 
       ad_build_rows(c, A, half_dt, d_fu, d_fv, d_fw);
     }
     if (fresh)
-      k_fresh_rhs<<<(3 * c->fr.n + 255) / 256, 256, 0, s>>>(c->fr.n, 3, c->fr.ids, c->fr.ids_s, nullptr, nullptr, fc);
+      k_fresh_rhs<<<(3 * c->fr.n + 255) / 256, 256, 0, s>>>(c->fr.n, 3, c->d_iblank_ref, c->fr.ids, c->fr.ids_s,
+                                                            nullptr, nullptr, fc);
     rc = ad_residual<3>(c, A, nullptr);
     if (rc) break;
     int qm = 0;

@@ -2588,18 +2588,21 @@ __global__ void k_fresh_ad_coef(int n, const long *__restrict__ ids, const doubl
 // in stencil order), from the fields as the pass starts, so every line of
 // the pass reads the same values.  var and rw are the momentum solve's split
 // rows (offsets ids_s, coff), r the caller's fields (offsets ids); coff null:
-// rw = r alone.  One thread per cell and field.
+// rw = r alone.  A blank cell that the mask marks (ib not 0) keeps its row.
+// One thread per cell and field.
 struct FreshCorr {
   const double *var[3];
   const double *r[3];
   double *rw[3];
 };
-__global__ void k_fresh_rhs(int n, int nv, const long *__restrict__ ids, const long *__restrict__ ids_s,
-                            const long *__restrict__ coff, const double *__restrict__ cc, FreshCorr F) {
+__global__ void k_fresh_rhs(int n, int nv, const int8_t *__restrict__ ib, const long *__restrict__ ids,
+                            const long *__restrict__ ids_s, const long *__restrict__ coff,
+                            const double *__restrict__ cc, FreshCorr F) {
 #pragma clang fp contract(off)
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n * nv) return;
   const int q = t % n, f = t / n;
+  if (ib[ids[q]]) return;
   const double *var = F.var[f];
   double s = 0.0;
   if (coff) {
