@@ -2309,7 +2309,13 @@ int time_kernel(pp_ctx *c, int cls, int level, int reps, double *avg_us, double 
   // the line passes of the FP32 level 0 run on its colour-split copy, as
   // in the mixed solve
   c->sp.on = std::is_same<T, float>::value && level == 0 && c->sp.ok && cls != PP_K_RESIDUAL;
+  const SmoothBuf<T> buf(c, level);
+  const bool pair = cls != PP_K_RESIDUAL && pair_level<T>(c, L, split_on<T>(c, level));
   for (int r = 0; r < reps; r++) {
+    if (pair) {
+      launch_pair<T>(c, level, cls - PP_K_XLINE, buf.b[r & 1], buf.b[1 - (r & 1)], T(1));
+      continue;
+    }
     switch (cls) {
       case PP_K_XLINE: launch_xline<T>(c, L, level, r & 1, T(1)); break;
       case PP_K_YLINE: launch_yzline<T, 1>(c, L, level, r & 1, T(1)); break;
