@@ -313,8 +313,13 @@ void launch_yzline(pp_ctx *c, Level &L, int lvl, int color, T omega) {
   kbegin(c, DIR == 1 ? PP_K_YLINE : PP_K_ZLINE, lvl, 0.5 * (double)L.cx * L.cy * L.cz * bytes_line(sizeof(T)));
   auto go = [&](auto ls) {
     constexpr int LS = decltype(ls)::value;
-    if (spl) k_yzline<T, LS, DIR, true><<<grid, block, lds, st>>>(a, hp, rhs, e, color, omega);
-    else k_yzline<T, LS, DIR, false><<<grid, block, lds, st>>>(a, hp, rhs, e, color, omega);
+    if constexpr (std::is_same<T, float>::value) {
+      if (spl) {
+        k_yzline<T, LS, DIR, true><<<grid, block, lds, st>>>(a, hp, rhs, e, color, omega);
+        return;
+      }
+    }
+    k_yzline<T, LS, DIR, false><<<grid, block, lds, st>>>(a, hp, rhs, e, color, omega);
   };
   using std::integral_constant;
   switch (sh.LS) {
