@@ -1837,7 +1837,7 @@ int32_t pp_destroy(pp_ctx *c) {
   hipFree(c->d_p); hipFree(c->d_b); hipFree(c->d_w); hipFree(c->d_bwork); hipFree(c->d_tmp);
   hipFree(c->d_fresh); hipFree(c->d_iblank_ref); hipFree(c->d_count); hipFree(c->d_mu); hipFree(c->d_sv);
   hipFree(c->d_ad_coef);
-  hipFree(c->adw.buf);
+  hipFree(c->d_adw);
   hipFree(c->d_nshape32); hipFree(c->d_nshape64);
   free_fresh_rows(c);
   hipFree(c->d_part); hipFree(c->d_part2); hipFree(c->d_res); hipFree(c->d_kcoef); hipFree(c->d_redcount);
@@ -2051,7 +2051,7 @@ AdSplit ad_split(const pp_ctx *c) {
   A.sx = SPLIT_E0 + 2 * A.hp;
   A.sxy = (long)A.sx * (c->nyc + 2);
   A.total = A.sxy * (c->nzc + 2);
-  double *b = c->adw.buf;
+  double *b = c->d_adw;
   for (int q = 0; q < 3; q++) { A.var[q] = b + q * A.total; A.rw[q] = b + (3 + q) * A.total; }
   A.row = b + 6 * A.total;
   return A;
@@ -2744,16 +2744,16 @@ FracMetrics ref_metrics(const pp_ctx *c) {
   return M;
 }
 
-// The working copy, allocated at the first call: every value an identity row
-// (coefficients 0, diagonal 1, right-hand side 0) until a solve writes its
-// interior cells.
+// The working copy, allocated where there is none: every value an identity
+// row (coefficients 0, diagonal 1, right-hand side 0) until a solve writes
+// its interior cells.
 int ad_work(pp_ctx *c, AdSplit *out) {
   AdSplit A = ad_split(c);
-  if (!c->adw.buf) {
-    HIPCHK(hipMalloc(&c->adw.buf, sizeof(double) * 13 * (size_t)A.total));
+  if (!c->d_adw) {
+    HIPCHK(hipMalloc(&c->d_adw, sizeof(double) * 13 * (size_t)A.total));
     A = ad_split(c);
     const unsigned nb = 4096;
-    k_fill<double><<<nb, 256, 0, c->stream>>>(c->adw.buf, 12 * A.total, 0.0);
+    k_fill<double><<<nb, 256, 0, c->stream>>>(c->d_adw, 12 * A.total, 0.0);
     k_fill<double><<<nb, 256, 0, c->stream>>>(A.row + 6 * A.total, A.total, 1.0);
     HIPCHK(hipGetLastError());
   }
@@ -3317,6 +3317,16 @@ int32_t pp_calc_residual_ad(pp_ctx *c, int32_t advec_scheme, const double *var, 
   const double *hin[5] = {var, r, fu, fv, fw};
   for (int q = 0; q < 5; q++) HIPCHK(hipMemcpy(dv[q], hin[q], nb, hipMemcpyHostToDevice));
   HIPCHK(hipMemsetAsync(dv[5], 0, nb, c->stream));
+  // one residual leaves no working copy behind
+  struct Work {
+    pp_ctx *c;
+    bool keep;
+    ~Work() {
+      if (keep) return;
+      hipFree(c->d_adw);
+      c->d_adw = nullptr;
+    }
+  } work{c, c->d_adw != nullptr};
   AdSplit A;
   rc = ad_work(c, &A);
   if (rc) return rc;

@@ -174,15 +174,6 @@ struct FreshRows {
   long *ids_s = nullptr, *coff_s = nullptr;  // ids and coff in the momentum solve's split rows
 };
 
-// The momentum solve's working copy (csrc/pp_momentum.h): u, v, w, their
-// masked right-hand sides and the seven row coefficients in colour-split
-// rows, allocated at the first momentum call and kept with the context.
-struct AdWork {
-  int hp = 0, sx = 0;
-  long sxy = 0, total = 0;     // values per array
-  double *buf = nullptr;       // 13 arrays of total values: var 3, rw 3, row 7
-};
-
 // the colour-split copy of level 0 used by the FP32 V-cycles, forward and
 // transposed (flags, correction, right-hand side, null-space shape; the
 // level-0 FP32 arrays stay in the natural layout for everything else)
@@ -250,7 +241,10 @@ struct pp_ctx {
   double ad_dt = 0.0;
   bool have_ad = false;
   pp::FreshRows fr;                    // fresh-cell rows of the current geometry
-  pp::AdWork adw;                      // working copy of the momentum solve
+  // the momentum solve's working copy (csrc/pp_momentum.h): u, v, w, their masked
+  // right-hand sides and the seven row coefficients in colour-split rows,
+  // allocated at the first pp_solve_ad and kept with the context
+  double *d_adw = nullptr;
   int null_iters = 0;
   double null_res = 0.0;           // level-0 smoother uses the transposed ghost rows
   std::vector<double *> d_kry;         // flexible GMRES (FP64 path): m+1 basis + m preconditioned vectors
