@@ -274,12 +274,24 @@ void launch_xline(pp_ctx *c, Level &L, int lvl, int color, T omega, bool zero = 
 // rows): LS cells per thread, P segments, TX lines per block (at most 1024
 // threads in FP32, 512 in FP64, whose segments take twice the registers).
 // A wide tile is one 128-byte line of a half row.  Longer segments cost fewer
-// reduction steps and barriers per cell, so LS is the longest that fills the
-// block and still lets the level's blocks be resident at once or nearly so:
-// 12 up to 192 cells (256x192x192 15.6 us; 16: 18.9, 8: 16.7), 16 beyond
-// (384x256x256 42 us; 8: 43, 12: 47; 512-cell lines 245; 8 in 16-line tiles
-// 262).  Levels of few blocks are latency-bound and get 8-line tiles of short
-// segments (128x96x96: 4 cells 6.3 us, 6 cells 6.6, 8 cells 6.9).
+// reduction steps and barriers per cell, but fewer threads per line; several
+// blocks share a CU while a tile's segments fit 512 threads (FP32; 256 in
+// FP64), so LS steps up where they no longer do: past 128 and 192 cells.  y
+// passes of 256 x n x 256 cells, us back to back (pp_time_kernel) with LS = 8,
+// 12, 16, the FP32 level in colour-split rows, the FP64 one in natural rows:
+//   n     FP32                FP64
+//   128   13.4  16.8  13.3    40.2  42.8  40.9
+//   130   19.4  17.4  19.2    51.1  43.0  47.6
+//   160   21.5  18.8  21.1    59.0  50.1  55.1
+//   192   20.2  20.6  23.9    71.2  61.0  62.2
+//   193   43.5  40.7  36.3    70.1  78.7  63.9   (natural rows in FP32 too)
+//   208   29.0  28.6  21.1    75.5  87.2  67.6
+// and 384x256x256 50.8, 48.5, 36.7 and 166, 196, 166; 512x512x384 (12 in
+// 16-line tiles, 8 in 16) 302, 296, 221 and 782, 933, 720.  Levels of few
+// blocks are latency-bound and get 8-line tiles of short segments (FP32, 4
+// cells, against LS = 8 in 32-line tiles: 64x48x48 3.5 and 4.1 us; 128x64x64
+// 4.2 and 4.4; but 128x96x96 5.8 and 5.1, 128x96x256 10.4 and 7.1: the
+// limit of 2048 blocks is higher than the FP32 figures alone ask for).
 struct YZShape {
   int LS, P, TX;
 };

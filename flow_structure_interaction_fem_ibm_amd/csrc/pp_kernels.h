@@ -620,7 +620,8 @@ __global__ void __launch_bounds__(NT) k_face_vel(RefArgs R, LevelArgs<double> L0
 // sweep to sweep in base; the later ones add the ghost-ghost entries alone,
 // and the last writes the fields (and u2, v2, w2 where given), which no
 // sweep but the first reads at a ghost.  Latency-bound (11k ghosts): 8 sweeps
-// 31 us against 73 with one lane per ghost and a gather and a scatter launch.
+// 40 us in a kernel trace (5.9 for the first, 4.9 each after it) against 74
+// with one lane per ghost and a gather and a scatter launch.
 struct VelGhostOut {
   const long *gref;            // field offset of each ghost; u null: the iterate buffer instead
   double *u, *v, *w, *u2, *v2, *w2;
@@ -1628,9 +1629,12 @@ __device__ inline int xcd_block(int b, int nb) {
 // cells and the S/2 odd cells beside them, read whole (the rows' padding and
 // the coefficients' run past the line's end).  Its faces are closed on the
 // outer boundary only, where the coefficients are 0, so its rows test the
-// blank flag alone; rows are chosen by selects, without branches: 256x192x192
-// 16.6 us per colour pass (FP64 32.1) against 20.6 (41.7) with a branch per
-// cell and flag, 467 against 917 VALU instructions per wavefront.
+// blank flag alone; rows are chosen by selects, without branches: 467 against
+// 917 VALU instructions per wavefront with a branch per cell and flag, and per
+// colour pass, back to back, 256x192x192 14.4 us against 18.6, 384x256x256 36.6
+// against 43.7, but 512x512x384 (S = 16, few wavefronts) 191 against 176; FP64
+// and odd rows, natural layout with selects per flag: 34.7 against 33.2 at
+// 256x192x192, 97 against 99 at 384x256x256.
 template <typename T, int G, int S, bool SPL = false>
 __global__ void __launch_bounds__(256) k_xline(LevelArgs<T> L, const T *__restrict__ rhs, T *__restrict__ e,
                                                int color, T omega, int hp, bool zero) {
@@ -1825,11 +1829,14 @@ __device__ inline void seg_reduced_solve(RedEq<T> *sh, int P, int tx, int seg, S
 // segment first, and the registers that takes cost more blocks per CU than
 // the extra loads in flight are worth (six wavefronts per SIMD hold three
 // 512-thread blocks of 12-cell segments: 83 registers instead of 80 cost
-// 11%).  Rows are chosen by selects.  One
-// colour pass on the split level, FP32: 256x192x192 15.6 us in y, 16.0 in z
-// (LS = 12, PF = 2, 32-line tiles) against 20.6 and 20.8 with a branch per
-// flag, LS = 8 and cells four ahead; 384x256x256 42 and 43 (LS = 16, PF = 4)
-// against 65 and 67; FP64 256x192x192 33.6 against 57 in natural rows.
+// 11%; held to 80 the kernel spills three or four, 4.6-6.3 MB more written per
+// launch).  Rows are chosen by selects.  One colour pass in y and z, back to
+// back, against the pass with a branch per flag, LS = 8 and cells four ahead:
+// FP32, split level, 256x192x192 (LS = 12, PF = 2, 32-line tiles) 16.5 and 17.2
+// us against 19.1 and 19.3 (17.8 and 18.0 within a solve), 384x256x256 (LS =
+// 16, PF = 4) 36.9 and 37.2 against 45.0 and 47.1, 512x512x384 221 and 229
+// against 333 and 256; FP64, natural rows, 256x192x192 46.5 and 48.3 against
+// 57.6 and 56.1.
 // ---------------------------------------------------------------------
 template <typename T, int LS>
 constexpr int yz_prefetch() { return LS <= 4 ? LS : (LS == 8 ? 4 : (LS == 16 && sizeof(T) == 4 ? 4 : 2)); }
